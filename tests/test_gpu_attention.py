@@ -141,6 +141,25 @@ def test_large_scores_and_scale(pkg, dev):
             assert torch.equal(pre, attn(q, k, vt, pos0, L, cps, True, scale))
 
 
+@pytest.mark.parametrize("B,T,H,KVH,D,scale,note", [
+    (8, 181, 40, 8, 128, None, "two row tiles per wave, a ragged last workgroup"),
+    (8, 181, 40, 8, 64, -0.2, "the same at D = 64, a negative scale"),
+    (3, 130, 10, 1, 128, None, "3 pairs: row groups dealt over all pairs"),
+    (2, 65, 4, 4, 64, 0.0, "a zero scale: every attended position weighs the same"),
+])
+def test_prefill_tiles_pairs_and_scales(pkg, dev, B, T, H, KVH, D, scale, note):
+    """Row tiles per wave, pair counts and signs of the scale: the reference on the first
+    sequence, and the bits of the split launch on every row."""
+    say(f"attention B={B} T={T} H={H} KVH={KVH} D={D} scale={scale} ({note})")
+    q, k, vt, Lc = make_inputs(dev, B, T, H, KVH, D, T, seed=T + D, q_scale=4.0)
+    pos0 = torch.zeros((1,), dtype=torch.int64, device=dev)
+    for cps in (1, Lc // 64):
+        pre = attn(q, k, vt, pos0, T, cps, False, scale)
+        ref, mag = reference(q[:1], k[:1], vt[:1], 0, T, scale)
+        check(pre[:1], ref, mag, f"cps={cps}")
+        assert torch.equal(pre, attn(q, k, vt, pos0, T, cps, True, scale)), f"split launch differs (cps={cps})"
+
+
 def test_positions_clamp_to_cache(pkg, dev):
     """pos[0] + t past L - 1 attends to the whole cache, a negative position to position 0."""
     B, H, KVH, D, L = 2, 8, 2, 64, 100

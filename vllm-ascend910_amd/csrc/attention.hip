@@ -14,17 +14,22 @@
 // Arithmetic of a row, in chunks of 64 positions:
 //   scores  S^T = K . Q^T by v_mfma_f32_16x16x32_bf16 (keys as the A rows, the
 //           16 query rows of a tile as the B columns) in fp32, times
-//           c = log2(e) * scale; positions past p(r) are -inf;
+//           c = log2(e) * |scale| (a negative scale flips the queries' signs
+//           instead, exact); positions past p(r) are -inf;
 //   chunk   flash update of the running state (m, l, O) of the split the
 //           chunk belongs to: m' = max(m, max_k s), alpha = 2^(m - m'),
-//           P = 2^(s - m'), l' = l * alpha + sum_k P, O' = O * alpha +
-//           bf16(P) . V (MFMA: V^T as the A rows, P^T as the B columns);
+//           P = 2^(s - m') (s - m' as one fused multiply-add of the score),
+//           l' = l * alpha + sum_k P, O' = O * alpha + bf16(P) . V (MFMA: V^T
+//           as the A rows, P^T as the B columns).  l is held per lane (each
+//           of a row's four lanes sums its own 16 positions of a chunk) and
+//           the four meet once, when the split ends;
 //   splits  `cps` consecutive chunks form a split; split states are combined
 //           in the order s = 0, 1, ... by (m1, l1, O1) (+) (m2, l2, O2) =
 //           (m, l1 a1 + l2 a2, O1 a1 + O2 a2), m = max(m1, m2), a_i = 2^(m_i - m);
 //   output  bf16(O * (1 / l)).
-// Every sum runs in an order that does not depend on which other rows share
-// a tile, so a row's result depends only on its query, the cache and cps: the
+// Every sum and every choice is made per row, in an order that does not depend
+// on which other rows share a tile, so a row's result depends only on its
+// query, the cache and cps: the
 // decode launch (one single-wave workgroup per split, the chunk operands
 // loaded straight into registers one chunk ahead, split states through a
 // workspace, then a combine kernel) and the prefill launch (four waves share
@@ -34,6 +39,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "launch.h"
@@ -75,7 +81,8 @@ struct VOps {
 };
 
 // Running state of one query row.  The row's four lanes (c, j = 0..3) each
-// hold m and l and the slice O^T[16 dt + 4 j + e][c], e = 0..3, of its O.
+// hold m, their share of l (all of it after state_close) and the slice
+// O^T[16 dt + 4 j + e][c], e = 0..3, of its O.
 template <int D>
 struct RowState {
     float m, l;
@@ -103,6 +110,31 @@ __device__ __forceinline__ void fold_coeffs(float m1, float m2, float& mn, float
 __device__ __forceinline__ float fold_value(float x1, float a1, float x2, float a2) {
 #pragma clang fp contract(off)
     return fmaf(x1, a1, x2 * a2);
+}
+
+// 2^x of a non-positive x: v_exp_f32 alone, results below 2^-126 as 0.
+__device__ __forceinline__ float exp2_neg(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// The larger of two, NaN if either is (v_maximum3_f32: unlike fmaxf it needs
+// no canonicalising move per MFMA result).
+__device__ __forceinline__ float vmax(float x, float y) { return __builtin_elementwise_maximum(x, y); }
+
+// The four lanes of a row (lane ^ 16, lane ^ 32) reduced by the gfx950 lane
+// swaps: x against itself gives one register holding the even and one holding
+// the odd 16-lane (32-lane) halves, so no LDS permute and no wait.
+template <class F>
+__device__ __forceinline__ float row_reduce(float x, F f) {
+    const uint32_t u = __float_as_uint(x);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const uint32_t v = __float_as_uint(f(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// The end of a split: l of the row's four lanes added.
+template <int D>
+__device__ __forceinline__ void state_close(RowState<D>& s) {
+    s.l = row_reduce(s.l, [](float p, float q) { return p + q; });
 }
 
 // s = s (+) t; an empty state (l == 0: no position of the row in that split) is
@@ -157,6 +189,11 @@ __device__ __forceinline__ int last_pos(const AttnArgs& a, int64_t pos0, int r1)
     return clamp_pos(pos0 + min(r1, a.G * a.T - 1) / a.G, a.L);
 }
 
+// Eight bf16 with their signs flipped where flip is 0x80008000 (0: unchanged).
+__device__ __forceinline__ uint4 flip_sign(uint4 v, uint32_t flip) {
+    return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip);
+}
+
 // Q^T as the B operand of the score MFMAs: lane (c, j) holds q[r][32 i + 8 j .. +8]
 // for k-step i; rows past the problem read zero.
 template <int D>
@@ -165,7 +202,7 @@ __device__ __forceinline__ void load_q(const AttnArgs& a, const Tile& t, int j, 
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) {
         const uint4 v = t.real ? *reinterpret_cast<const uint4*>(qr + 32 * i + 8 * j) : make_uint4(0, 0, 0, 0);
-        qop[i] = __builtin_bit_cast(bf16x8, v);
+        qop[i] = __builtin_bit_cast(bf16x8, flip_sign(v, a.qflip));
     }
 }
 
@@ -205,40 +242,39 @@ __device__ __forceinline__ void chunk_scores(f32x4 (&sc)[4], const bf16x8 (&qop)
     }
 }
 
-// The softmax update and the output product of one chunk (positions c0 ..).
-template <int D>
-__device__ __forceinline__ void chunk_update(RowState<D>& st, const f32x4 (&sc)[4], const VOps<D>& vo, int c0,
-                                             int p_row, float cs, int j) {
+// The softmax update of one chunk (positions c0 ..): m and l of the state, the
+// factor alpha of its O, and P^T as the B operands of the chunk's two key
+// blocks.  MASK: the chunk may hold positions past p_row.  cs > 0.
+template <bool MASK>
+__device__ __forceinline__ void chunk_softmax(float& m, float& l, float& alpha, bf16x8 (&pop)[2],
+                                              const f32x4 (&sc)[4], int c0, int p_row, float cs, int j) {
 #pragma clang fp contract(off)
-    float x[4][4];
-    float mloc = -INFINITY;
+    float x[4][4], mt[4];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x[kt][e] = c0 + lane_pos(kt, j, e) <= p_row ? sc[kt][e] * cs : -INFINITY;
-            mloc = fmaxf(mloc, x[kt][e]);
-        }
-    float mc = fmaxf(mloc, __shfl_xor(mloc, 16));
-    mc = fmaxf(mc, __shfl_xor(mc, 32));
-    const float mn = fmaxf(st.m, mc);
+        for (int e = 0; e < 4; ++e)
+            x[kt][e] = (!MASK || lane_pos(kt, 0, e) <= p_row - c0 - 8 * j) ? sc[kt][e] : -INFINITY;
+        mt[kt] = vmax(vmax(x[kt][0], x[kt][1]), x[kt][2]);
+    }
+    mt[0] = vmax(vmax(mt[0], x[0][3]), x[1][3]);
+    mt[2] = vmax(vmax(mt[2], x[2][3]), x[3][3]);
+    mt[0] = vmax(vmax(mt[0], mt[1]), vmax(mt[2], mt[3]));
+    const float xm = row_reduce(mt[0], [](float p, float q) { return vmax(p, q); }) * cs;
+    const float mn = vmax(m, xm);
     const float mz = mn == -INFINITY ? 0.0f : mn;   // no position of the row yet: everything stays 0
-    const float alpha = exp2f(st.m - mz);
-    float p[4][4];
-    float lsum = 0.0f;
+    // an empty state needs no factor (its l and O are 0)
+    alpha = m != -INFINITY ? exp2_neg(m - mz) : 1.0f;
+    float p[4][4], ls[4];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            p[kt][e] = exp2f(x[kt][e] - mz);
-            lsum = lsum + p[kt][e];
-        }
-    lsum = lsum + __shfl_xor(lsum, 16);
-    lsum = lsum + __shfl_xor(lsum, 32);
-    st.l = fmaf(st.l, alpha, lsum);
-    st.m = mn;
+        for (int e = 0; e < 4; ++e) p[kt][e] = exp2_neg(fmaf(x[kt][e], cs, -mz));
+        ls[kt] = (p[kt][0] + p[kt][1]) + (p[kt][2] + p[kt][3]);
+    }
+    l = fmaf(l, alpha, (ls[0] + ls[1]) + (ls[2] + ls[3]));
+    m = mn;
     // P^T as the B operand of key block s: slots 0..7 = positions 32 s + 8 j + 0..7
-    bf16x8 pop[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const uint4 w = make_uint4(f32x2_to_bf16x2_bits(p[2 * s][0], p[2 * s][1]),
@@ -247,13 +283,32 @@ __device__ __forceinline__ void chunk_update(RowState<D>& st, const f32x4 (&sc)[
                                    f32x2_to_bf16x2_bits(p[2 * s + 1][2], p[2 * s + 1][3]));
         pop[s] = __builtin_bit_cast(bf16x8, w);
     }
+}
+
+// O *= alpha; nothing where no row of the wave's tile has a new maximum (alpha = 1
+// keeps every bit).
+template <int D>
+__device__ __forceinline__ void state_scale(RowState<D>& st, float alpha) {
+#pragma clang fp contract(off)
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) == 0) return;
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) {
+    for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) st.o[dt][e] = st.o[dt][e] * alpha;
+}
+
+// The softmax update and the output product of one chunk (positions c0 ..).
+template <int D>
+__device__ __forceinline__ void chunk_update(RowState<D>& st, const f32x4 (&sc)[4], const VOps<D>& vo, int c0,
+                                             int p_row, float cs, int j) {
+    float alpha;
+    bf16x8 pop[2];
+    chunk_softmax<true>(st.m, st.l, alpha, pop, sc, c0, p_row, cs, j);
+    state_scale(st, alpha);
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
         for (int s = 0; s < 2; ++s) st.o[dt] = mfma_bf16(__builtin_bit_cast(bf16x8, vo.v[dt][s]), pop[s], st.o[dt]);
-    }
 }
 
 // bf16(O * (1 / l)) of the lane's slice of row r.
@@ -423,7 +478,7 @@ __global__ __launch_bounds__(64) void attn_split_kernel(const AttnArgs a) {
         rope_rotate<D>(xk, bk, has_bias, cs, sn, knew);
 #pragma unroll
         for (int i = 0; i < D / 32; ++i)
-            qop[i] = __builtin_bit_cast(bf16x8, (inside && t.real) ? yq[i] : make_uint4(0, 0, 0, 0));
+            qop[i] = __builtin_bit_cast(bf16x8, (inside && t.real) ? flip_sign(yq[i], a.qflip) : make_uint4(0, 0, 0, 0));
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt)
             vnew[dt] = has_bias ? f32_to_bf16_bits(rope_in(xv[dt], bv[dt], true)) : xv[dt];
@@ -484,6 +539,7 @@ __global__ __launch_bounds__(64) void attn_split_kernel(const AttnArgs a) {
         ++ch;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the skipped prefetch
+    state_close(st);
     if (a.ns == 1) {
         write_out<D>(a, t, st, j);
         return;
@@ -560,114 +616,167 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const AttnArgs a) {
     }
 }
 
-// Prefill launch: a workgroup of four waves takes 64 rows (four 16-row tiles)
-// of one pair and walks the chunks up to its last row's position; each chunk's
-// K and V^T (32 KB at D = 128) go from memory straight into one of two LDS
-// buffers, one chunk ahead, and every wave reads its operands from there.  Rows
-// of 2D (K) or 128 (V^T) bytes are stored with their 16-byte chunks permuted
-// (chunk q of row r at q ^ kswz(r) / q ^ vswz(r)) so that the operand reads of
-// eight consecutive lanes fall in distinct banks.  Workgroups are numbered so
-// that each XCD (workgroups go to the eight XCDs round-robin) takes a
-// contiguous run -- the row groups of a few pairs, whose K and V stay in that
-// XCD's L2 -- the row groups with the most positions first within each pair.
-constexpr int kLoopWaves = 4;
+// Prefill launch: a workgroup of four waves takes 64 RT rows (RT 16-row tiles
+// per wave) of one pair and walks the chunks up to its last row's position;
+// each chunk's K and V^T (16 KB each at D = 128) go from memory straight into
+// one of two LDS buffers, one chunk ahead, and every wave reads its operands
+// from there, each read serving the wave's RT tiles.  Rows of 2D (K) or 128
+// (V^T) bytes are stored with their 16-byte chunks permuted (chunk q of row r at
+// q ^ kswz(r) / q ^ vswz(r)) so that the operand reads of sixteen consecutive
+// lanes fall in distinct banks.
+//
+// What bounds it: the vector instructions of the softmax.  Per 16-row tile and
+// chunk there are 32 MFMAs (16 cycles each) and about 80 vector instructions off
+// the diagonal (16 exponentials at two issue slots), 32 more where a row's
+// maximum moves; 40 heads of 128 over 8 KV heads, one sequence: 4096 tokens
+// 279 -> 195 us, 8192 tokens 704 us = 0.98 PFLOP/s where a large bf16 matrix
+// product reaches 1.19 on the same card.  What it took: two row tiles per wave
+// (one operand read serves two), masks only on the chunks that need them, lane
+// swaps instead of LDS permutes, the maximum on the raw scores and one fused
+// multiply-add per exponent.  Slower at 4096 tokens: the softmax of one tile
+// placed between the MFMAs of the other in one wave (235 us), eight waves of
+// one tile (202), the folded split states in scratch (233: its loads wait
+// behind the chunk prefetch).
 
+// Sixteen lanes read rows tile_row_pos(kt, 0..15) = 8 (c / 4) + (c % 4) + const at
+// one logical chunk: at D = 128 (16 chunks, one row spans every bank) the XOR is c
+// itself, at D = 64 (two rows span the banks) the three bits of c past its parity.
 template <int D>
 __device__ __forceinline__ int kswz(int r) {
-    return D == 128 ? (r & 15) : ((r >> 1) & 7);
+    return D == 128 ? ((r & 3) | ((r >> 1) & 12)) : (((r >> 1) & 1) | ((r >> 2) & 6));
 }
 __device__ __forceinline__ int vswz(int d) { return (d >> 1) & 7; }
 
-template <int D>
-__global__ __launch_bounds__(64 * kLoopWaves) void attn_loop_kernel(const AttnArgs a, int groups) {
-    constexpr int KB = kChunk * D * 2;               // K bytes of a chunk
-    constexpr int CB = 2 * KB;                       // K + V^T bytes of a chunk
-    constexpr int LPT = CB / (64 * kLoopWaves * 16); // 16-byte loads per thread per chunk
-    constexpr int KLD = KB / (64 * kLoopWaves * 16); // ... of which K
+constexpr int kLoopWaves = 4;
+
+// Workgroup -> (pair, row group), the row groups with the most positions first.
+// Workgroups go to the eight XCDs round-robin.  Pairs in eighths: each XCD takes
+// a contiguous run, whole pairs one after the other, so K and V stay in its L2.
+// Other counts: row group by row group over all pairs, since a contiguous run
+// would give some XCDs only the long groups of a pair (2 pairs of 5 heads, 4096
+// tokens: 106 -> 67 us).
+__device__ __forceinline__ void loop_tile(int pairs, int groups, int& pair, int& grp) {
+    const int bid = static_cast<int>(blockIdx.x);
+    int rank;
+    if (pairs % 8 == 0) {
+        const int lin = (bid & 7) * (pairs / 8 * groups) + (bid >> 3);
+        pair = lin / groups;
+        rank = lin - pair * groups;
+    } else {
+        rank = bid / pairs;
+        pair = bid - rank * pairs;
+    }
+    grp = groups - 1 - rank;
+}
+
+template <int D, int RT>
+__global__ __launch_bounds__(64 * kLoopWaves, 2) void attn_loop_kernel(const AttnArgs a, int groups) {
+    constexpr int NW = kLoopWaves;
+    constexpr int KB = kChunk * D * 2;               // K (or V^T) bytes of a chunk
+    constexpr int LPT = KB / (64 * NW * 16);         // 16-byte loads per thread per chunk of each
     // two chunk buffers as two arrays (the loop is unrolled by two), so the compiler
     // sees that the loads into one never alias the operand reads from the other
-    __shared__ __attribute__((aligned(16))) char lds0[CB];
-    __shared__ __attribute__((aligned(16))) char lds1[CB];
+    __shared__ __attribute__((aligned(16))) char lds0[2 * KB];
+    __shared__ __attribute__((aligned(16))) char lds1[2 * KB];
     const int tid = static_cast<int>(threadIdx.x);
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int c = lane & 15, j = lane >> 4;
-    const int nwg = static_cast<int>(gridDim.x), bid = static_cast<int>(blockIdx.x);
-    const int xcd = bid & 7, q8 = nwg >> 3, rem = nwg & 7;
-    const int lin = xcd * q8 + min(xcd, rem) + (bid >> 3);
-    const int pair = lin / groups;
-    const int grp = groups - 1 - (lin - pair * groups);
-    const Tile t = make_tile<D>(a, pair, kLoopWaves * grp + wave, c);
-    const __amdgpu_buffer_rsrc_t kr = pair_rsrc(a.k, t.pair, a.Lc, D);
-    const __amdgpu_buffer_rsrc_t vr = pair_rsrc(a.vt, t.pair, a.Lc, D);
-    // this thread's loads: load n lands at LDS byte n * 4096 + 16 * tid of the buffer
-    uint32_t goff[LPT];
+    int pair, grp;
+    loop_tile(a.B * a.KVH, groups, pair, grp);
+    const int rt0 = (NW * grp + wave) * RT;          // the wave's first row tile
+    const __amdgpu_buffer_rsrc_t kr = pair_rsrc(a.k, pair, a.Lc, D);
+    const __amdgpu_buffer_rsrc_t vr = pair_rsrc(a.vt, pair, a.Lc, D);
+    // this thread's loads: load n lands at LDS byte n * 1024 NW + 16 * tid of the buffer
+    uint32_t kgo[LPT], vgo[LPT];
 #pragma unroll
     for (int n = 0; n < LPT; ++n) {
-        const int P = n * 64 * kLoopWaves * 16 + 16 * tid;
-        if (n < KLD) {
-            const int r = P / (2 * D), pq = (P % (2 * D)) / 16;
-            goff[n] = static_cast<uint32_t>(r * 2 * D + 16 * (pq ^ kswz<D>(r)));
-        } else {
-            const int P2 = P - KB;
-            const int d = P2 / 128, pq = (P2 % 128) / 16;
-            goff[n] = static_cast<uint32_t>(d * a.Lc * 2 + 16 * (pq ^ vswz(d)));
-        }
+        const int P = n * 64 * NW * 16 + 16 * tid;
+        const int r = P / (2 * D), rq = (P % (2 * D)) / 16;
+        kgo[n] = static_cast<uint32_t>(r * 2 * D + 16 * (rq ^ kswz<D>(r)));
+        const int d = P / 128, dq = (P % 128) / 16;
+        vgo[n] = static_cast<uint32_t>(d * a.Lc * 2 + 16 * (dq ^ vswz(d)));
     }
     // chunk ch into buf; a chunk past the last one reads zero (kSkip) without memory traffic
-    auto load_chunk = [&](int ch, char* buf, bool real) {
-        char* dst = buf + 1024 * wave;
-        const uint32_t skip = real ? 0u : kSkip;
+    auto load_chunk = [&](int ch, char* buf, bool real) __attribute__((always_inline)) {
+        const uint32_t ko = real ? static_cast<uint32_t>(ch * kChunk * 2 * D) : kSkip;
+        const uint32_t vo = real ? static_cast<uint32_t>(ch * kChunk * 2) : kSkip;
 #pragma unroll
-        for (int n = 0; n < LPT; ++n) {
-            if (n < KLD)
-                buf_load16_lds(kr, dst + n * 4096, static_cast<uint32_t>(ch * kChunk * 2 * D) + goff[n] + skip);
-            else
-                buf_load16_lds(vr, dst + n * 4096, static_cast<uint32_t>(ch * kChunk * 2) + goff[n] + skip);
-        }
+        for (int n = 0; n < LPT; ++n) buf_load16_lds(kr, buf + 1024 * wave + n * 1024 * NW, ko + kgo[n]);
+#pragma unroll
+        for (int n = 0; n < LPT; ++n) buf_load16_lds(vr, buf + KB + 1024 * wave + n * 1024 * NW, vo + vgo[n]);
     };
     load_chunk(0, lds0, true);
-    bf16x8 qop[D / 32];
-    load_q<D>(a, t, j, qop);
     const int64_t pos0 = a.pos[0];
-    const int p_row = clamp_pos(pos0 + t.tok, a.L);
-    const int nchunks = last_pos(a, pos0, kLoopWaves * 16 * grp + kLoopWaves * 16 - 1) / kChunk + 1;
-    // this lane's operand addresses inside a chunk buffer
-    uint32_t kaddr[4][D / 32], vaddr[D / 16][2];
+    const int nchunks = last_pos(a, pos0, NW * 16 * RT * (grp + 1) - 1) / kChunk + 1;
+    bf16x8 qop[RT][D / 32];
+    int p_row[RT];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int t = 0; t < RT; ++t) {
+        const Tile tl = make_tile<D>(a, pair, rt0 + t, c);
+        load_q<D>(a, tl, j, qop[t]);
+        p_row[t] = clamp_pos(pos0 + tl.tok, a.L);
+    }
+    // chunks before this one hold no position past any of the wave's rows
+    const int free_chunks = (clamp_pos(pos0 + rt0 * 16 / a.G, a.L) + 1) / kChunk;
+    // This lane's operand addresses inside a chunk buffer.  K tile kt, k-step i is
+    // row r = tile_row_pos(kt, c), logical chunk 4 i + j (the same permutation in
+    // every tile); V^T tiles are 16 rows apart, again with one permutation.
+    uint32_t kaddr[D / 32], vaddr[2];
 #pragma unroll
-        for (int i = 0; i < D / 32; ++i) {
-            const int r = tile_row_pos(kt, c);
-            kaddr[kt][i] = static_cast<uint32_t>(r * 2 * D + 16 * ((4 * i + j) ^ kswz<D>(r)));
+    for (int i = 0; i < D / 32; ++i) {
+        const int r = tile_row_pos(0, c);
+        kaddr[i] = static_cast<uint32_t>(r * 2 * D + 16 * ((4 * i + j) ^ kswz<D>(r)));
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) vaddr[s] = static_cast<uint32_t>(KB + c * 128 + 16 * ((4 * s + j) ^ vswz(c)));
+    RowState<D> st[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) state_clear(st[t]);
+    RowState<D> tot[RT];                             // the splits walked so far, folded
+#pragma unroll
+    for (int t = 0; t < RT; ++t) state_clear(tot[t]);
+    auto end_split = [&](int t, int ch) __attribute__((always_inline)) {
+        if ((ch + 1) % a.cps == 0 || ch + 1 == nchunks) {
+            state_close(st[t]);
+            state_fold<D>(tot[t], st[t]);
+            state_clear(st[t]);
         }
+    };
+    auto step = [&](const char* buf, int ch) __attribute__((always_inline)) {
+        f32x4 sc[RT][4];
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt)
+        for (int kt = 0; kt < 4; ++kt) {
+            bf16x8 ko[D / 32];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int d = 16 * dt + c;
-            vaddr[dt][s] = static_cast<uint32_t>(KB + d * 128 + 16 * ((4 * s + j) ^ vswz(d)));
+            for (int i = 0; i < D / 32; ++i)
+                ko[i] = *reinterpret_cast<const bf16x8*>(buf + kaddr[i] + tile_row_pos(kt, 0) * 2 * D);
+#pragma unroll
+            for (int t = 0; t < RT; ++t) sc[t][kt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+                for (int t = 0; t < RT; ++t) sc[t][kt] = mfma_bf16(ko[i], qop[t][i], sc[t][kt]);
         }
-    RowState<D> tot, st;
-    state_clear(tot);
-    state_clear(st);
-    auto step = [&](const char* buf, int ch) {
-        KOps<D> ko;
+        bf16x8 pop[RT][2];
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int i = 0; i < D / 32; ++i) ko.k[kt][i] = *reinterpret_cast<const uint4*>(buf + kaddr[kt][i]);
-        f32x4 sc[4];
-        chunk_scores<D>(sc, qop, ko);
-        VOps<D> vo;
+        for (int t = 0; t < RT; ++t) {
+            float alpha;
+            if (ch < free_chunks)
+                chunk_softmax<false>(st[t].m, st[t].l, alpha, pop[t], sc[t], ch * kChunk, p_row[t], a.cs, j);
+            else
+                chunk_softmax<true>(st[t].m, st[t].l, alpha, pop[t], sc[t], ch * kChunk, p_row[t], a.cs, j);
+            state_scale(st[t], alpha);
+        }
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) vo.v[dt][s] = *reinterpret_cast<const uint4*>(buf + vaddr[dt][s]);
-        chunk_update<D>(st, sc, vo, ch * kChunk, p_row, a.cs, j);
-        if ((ch + 1) % a.cps == 0 || ch + 1 == nchunks) {
-            state_fold<D>(tot, st);
-            state_clear(st);
-        }
+            for (int s = 0; s < 2; ++s) {
+                const bf16x8 vo = *reinterpret_cast<const bf16x8*>(buf + vaddr[s] + dt * 16 * 128);
+#pragma unroll
+                for (int t = 0; t < RT; ++t) st[t].o[dt] = mfma_bf16(vo, pop[t][s], st[t].o[dt]);
+            }
+#pragma unroll
+        for (int t = 0; t < RT; ++t) end_split(t, ch);
     };
     for (int ch = 0;;) {
         // chunk ch has landed (every wave's part); every wave is done with chunk ch - 1
@@ -681,7 +790,8 @@ __global__ __launch_bounds__(64 * kLoopWaves) void attn_loop_kernel(const AttnAr
         if (++ch >= nchunks) break;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load into LDS outlives the workgroup
-    write_out<D>(a, t, tot, j);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) write_out<D>(a, make_tile<D>(a, pair, rt0 + t, c), tot[t], j);
 }
 
 template <int D>
@@ -696,17 +806,31 @@ hipError_t launch_attention_d(const AttnArgs& a, bool split, hipStream_t stream)
         if (a.ns > 1)
             attn_combine_kernel<D><<<dim3(static_cast<unsigned>(pairs * R)), dim3(64), 0, stream>>>(a);
     } else {
-        const int groups = static_cast<int>((R + 16 * kLoopWaves - 1) / (16 * kLoopWaves));
-        attn_loop_kernel<D><<<dim3(static_cast<unsigned>(static_cast<int64_t>(pairs) * groups)),
-                              dim3(64 * kLoopWaves), 0, stream>>>(a, groups);
+        // Two row tiles per wave where that still gives every CU two workgroups; one
+        // below (40 heads, 1 sequence: 1024 tokens 36.5 / 24.0 us, 2048 68 / 68,
+        // 4096 195 / 214, 8 sequences of 1024 134 / 146, two tiles / one).
+        const int64_t g2 = (R + 32 * kLoopWaves - 1) / (32 * kLoopWaves);
+        const int64_t g1 = (R + 16 * kLoopWaves - 1) / (16 * kLoopWaves);
+        const dim3 block(64 * kLoopWaves);
+        if (pairs * g2 >= 2 * device_cu_count())
+            attn_loop_kernel<D, 2><<<dim3(static_cast<unsigned>(pairs * g2)), block, 0, stream>>>(
+                a, static_cast<int>(g2));
+        else
+            attn_loop_kernel<D, 1><<<dim3(static_cast<unsigned>(pairs * g1)), block, 0, stream>>>(
+                a, static_cast<int>(g1));
     }
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_attention(const AttnArgs& a, bool split, hipStream_t stream) {
-    if (static_cast<int64_t>(a.B) * a.T == 0) return hipSuccess;
+hipError_t launch_attention(const AttnArgs& a0, bool split, hipStream_t stream) {
+    if (static_cast<int64_t>(a0.B) * a0.T == 0) return hipSuccess;
+    AttnArgs a = a0;
+    a.qflip = a.cs < 0.0f ? 0x80008000u : 0u;
+    // a factor of 0 (every score 0) as the smallest normal one: the same scores, but
+    // a masked position's -inf stays -inf
+    a.cs = fmaxf(fabsf(a.cs), 1.17549435e-38f);
     if (a.D == 128) return launch_attention_d<128>(a, split, stream);
     return launch_attention_d<64>(a, split, stream);
 }

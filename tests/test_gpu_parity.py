@@ -120,6 +120,29 @@ def test_quant_byte_exact_odd_and_large_rows(pkg, dev, K):
     assert np.array_equal(a_q.cpu().numpy(), q_ref)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 255, 256])
+@pytest.mark.parametrize("K,group", [(8200, 0), (32768, 0), (32776, 0), (40000, 96)])
+def test_quant_split_rows_mixed_ties(dev, M, K, group):
+    """Long rows on every split of a row over workgroups (and the unsplit launch past them),
+    each wave holding a few exact half-way quotients among ordinary values; a row of zeros
+    (tiny scale) and one of infinities keep the element-by-element forms."""
+    say(f"quant split M={M} K={K} group={group}")
+    rng = np.random.default_rng(M + K)
+    xb = np.tile(tie_rows(8, 512, seed=M), (-(-M // 8), 1))[:M]
+    # ordinary values of the row's own range, ties sprinkled among them
+    amax = ow.bf16_bits_to_f32(xb & 0x7fff).max(1, keepdims=True)
+    big = ow.f32_to_bf16_bits((rng.uniform(-1, 1, (M, K)) * amax).astype(np.float32))
+    at = rng.choice(K, 512, replace=False)
+    big[:, at] = xb
+    if M > 16:
+        big[3], big[5] = 0, 0x7f80
+    a_q, a_s = torch.ops.npu.w4a8_quant_pertoken(bf16_bits_tensor(big).to(dev), group)
+    rows = np.arange(M) != (5 if M > 16 else M)
+    q_ref, s_ref = ow.quant_act_per_token(big[rows])
+    assert np.array_equal(tensor_bf16_bits(a_s)[rows], s_ref)
+    assert np.array_equal(a_q.cpu().numpy()[rows], ow.pad_groups(q_ref, group) if group else q_ref)
+
+
 def test_quant_ties_zero_rows_and_strided_input(dev):
     say("quant ties/zero/strided")
     xb = tie_rows(64, 512, seed=11)

@@ -508,9 +508,7 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
         uint32_t amax = 0u;
 #pragma unroll
         for (int i = 0; i < QW; ++i) amax = max(amax, abs_bits_max8(xw[i]));
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1)
-            amax = max(amax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(amax), off, 64)));
+        amax = wave_max(amax);
         amax = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(amax)));
         const uint32_t sbits = scale_from_amax(amax);
         const bool writer = cgi == 0 && rgi == 0;   // one workgroup emits a_q / a_scale
@@ -521,23 +519,17 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
         const RowScale q = row_scale(bf16_bits_to_f32(sbits));
         // quantise this wave's own K range into its part of the LDS row
         const int c0 = k0 >> 3, c1 = k1 >> 3;
-        auto emit = [&](auto fast) __attribute__((always_inline)) {
-            constexpr bool F = decltype(fast)::value;
 #pragma unroll
-            for (int i = 0; i < QW; ++i) {
-                const int c = lane + 64 * i;
-                if (c >= c0 && c < c1) {
-                    const uint4 v = xw[i];
-                    uint2 o;
-                    o.x = quant2<F>(v.x, q) | (quant2<F>(v.y, q) << 16);
-                    o.y = quant2<F>(v.z, q) | (quant2<F>(v.w, q) << 16);
-                    *reinterpret_cast<uint2*>(lds + lq_a + 8 * c) = o;
-                    if (writer) *reinterpret_cast<uint2*>(p.aq_out + 8 * c) = o;
-                }
+        for (int i = 0; i < QW; ++i) {
+            // chunks 64 i .. 64 i + 63 hold none of the wave's range: a wave-uniform skip
+            if (64 * i + 64 <= c0 || 64 * i >= c1) continue;
+            const int c = lane + 64 * i;
+            const uint2 o = quant_unit(xw[i], q);
+            if (c >= c0 && c < c1) {
+                *reinterpret_cast<uint2*>(lds + lq_a + 8 * c) = o;
+                if (writer) *reinterpret_cast<uint2*>(p.aq_out + 8 * c) = o;
             }
-        };
-        if (q.fast) emit(std::true_type{});
-        else emit(std::false_type{});
+        }
     } else if constexpr (QF) {
         uint32_t am[QM];
 #pragma unroll
@@ -545,9 +537,7 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
             am[m] = 0u;
 #pragma unroll
             for (int i = 0; i < QI; ++i) am[m] = max(am[m], abs_bits_max8(xv[m][i]));
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1)
-                am[m] = max(am[m], static_cast<uint32_t>(__shfl_xor(static_cast<int>(am[m]), off, 64)));
+            am[m] = wave_max(am[m]);
         }
         if (lane == 0) {
 #pragma unroll
@@ -561,9 +551,7 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
             if (m >= p.M) break;
             // lane w < kw reads wave w's absmax, then a wave-wide max
             uint32_t amax = lane < kw ? reinterpret_cast<const uint32_t*>(lds + lq_m)[lane * 4 + m] : 0u;
-#pragma unroll
-            for (int off = 8; off >= 1; off >>= 1)
-                amax = max(amax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(amax), off, 64)));
+            amax = wave_max(amax);
             amax = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(amax)));
             const uint32_t sbits = scale_from_amax(amax);
             if (wave == 0 && lane == 0) {
@@ -571,23 +559,16 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
                 if (writer) p.as_out[m] = static_cast<uint16_t>(sbits);
             }
             const RowScale q = row_scale(bf16_bits_to_f32(sbits));
-            auto emit = [&](auto fast) __attribute__((always_inline)) {
-                constexpr bool F = decltype(fast)::value;
 #pragma unroll
-                for (int i = 0; i < QI; ++i) {
-                    const int c = lane + 64 * i;
-                    if (i < p.qcpr && c < nch) {
-                        const uint4 v = xv[m][i];
-                        uint2 o;
-                        o.x = quant2<F>(v.x, q) | (quant2<F>(v.y, q) << 16);
-                        o.y = quant2<F>(v.z, q) | (quant2<F>(v.w, q) << 16);
-                        *reinterpret_cast<uint2*>(lds + lq_a + m * p.lrs + k0 + 8 * c) = o;
-                        if (writer) *reinterpret_cast<uint2*>(p.aq_out + m * p.lda_out + k0 + 8 * c) = o;
-                    }
+            for (int i = 0; i < QI; ++i) {
+                if (i >= p.qcpr) break;
+                const int c = lane + 64 * i;
+                const uint2 o = quant_unit(xv[m][i], q);
+                if (c < nch) {
+                    *reinterpret_cast<uint2*>(lds + lq_a + m * p.lrs + k0 + 8 * c) = o;
+                    if (writer) *reinterpret_cast<uint2*>(p.aq_out + m * p.lda_out + k0 + 8 * c) = o;
                 }
-            };
-            if (q.fast) emit(std::true_type{});
-            else emit(std::false_type{});
+            }
         }
     }
     if (busy) {

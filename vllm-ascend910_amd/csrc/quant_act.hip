@@ -8,13 +8,13 @@
 // The quotient is the IEEE divide's (the reference kernel insists on it,
 // npu_ops/kernel/midgroup_quant_a.inc:55-62): a plain reciprocal multiply
 // would flip half-way cases relative to torch.  The codes here come from a
-// reciprocal multiply plus an exact half-way test (RowScale, common.h) that gives
+// reciprocal multiply plus an exact half-way test (RowScale, quant_unit, common.h) that gives
 // the divide's result for every input; rows whose scale is not a normal
 // float divide per element.
 //
 // Layout: one workgroup per row (256 threads, 1024 for rows longer than 8192
 // elements, so a decode-sized call still has enough loads in flight; long
-// rows of a small batch are split into 1024-thread chunks).  The row is read
+// rows of a small batch are split over several workgroups).  The row is read
 // once with 16-byte loads into registers, |x| is reduced as integers (for
 // finite bf16 the magnitude order equals the order of the 15 low bits), then
 // the same registers are quantised and written back as 8-byte int8 stores.
@@ -24,8 +24,6 @@
 // activation planes in the same padded layout, midgroup_quant_a.inc:7-12):
 // code k goes to (k / group) * stride + k % group, and the padding slots of
 // every group are written as zero.
-#include <type_traits>
-
 #include "common.h"
 #include "kgeom.h"
 #include "launch.h"
@@ -38,8 +36,7 @@ constexpr int kThreads = 256;
 // Block-wide max of a uint32 over NT threads.
 template <int NT>
 __device__ __forceinline__ uint32_t block_max(uint32_t v, uint32_t* red) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, 64)));
+    v = wave_max(v);
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) red[wave] = v;
     __syncthreads();
@@ -78,56 +75,59 @@ __device__ __forceinline__ void zero_pads(int8_t* qr, int K, const PadMap& pm) {
 }
 
 // Vector path: K % 8 == 0, rows 16-byte aligned; with PAD also group % 8 == 0
-// (an 8-code unit never straddles a group).  A workgroup quantises the
-// 16-byte units [blockIdx.y * cv, +cv) of its row (at most VPT * NT), held in
-// registers; with SPLIT (long rows of small batches, gridDim.y > 1) it also
-// reads the rest of the row for the absmax, so each chunk's workgroup finds
-// the same scale and the per-element work spreads over gridDim.y CUs.
+// (an 8-code unit never straddles a group).  A workgroup holds its row in
+// registers as 16-byte units, unit t + i NT in thread t.  With SPLIT (long rows of
+// small batches) gridDim.y workgroups share a row: each reads all of it for the
+// absmax, every load in flight at once, and quantises the units of i = blockIdx.y,
+// so the per-element work spreads over gridDim.y CUs.  Rows past VPT * NT units
+// (SPLIT only) are read in a loop instead, and the workgroup's own units again.
+//
+// Bound by memory on many rows (16384 x 27648: 259 -> 231 us, 5.9 TB/s of its 1.36
+// GB, from five instead of fourteen vector instructions per element) and by
+// latency on few: one memory round trip, two block-wide steps and the per-element
+// work of a thread's units (1 x 5120 3.1 -> 2.6 us in a graph of back-to-back calls).
 template <int VPT, int NT, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(NT) void quant_act_vec_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int8_t* __restrict__ aq, int64_t lda,
-    uint16_t* __restrict__ ascale, int K, const PadMap pm, int cv) {
+    uint16_t* __restrict__ ascale, int K, const PadMap pm) {
     __shared__ uint32_t red[NT / 64];
     const int64_t row = blockIdx.x;
-    const uint4* xr = reinterpret_cast<const uint4*>(x + row * ldx);
+    // buffer loads (units past the row read zero): under a branch each load is
+    // followed by register copies that wait for it before the next is issued
+    const auto xr = make_rsrc(x + row * ldx, static_cast<uint32_t>(K) * 2u);
     const int nvec = K >> 3;
-    const int v0 = SPLIT ? static_cast<int>(blockIdx.y) * cv : 0;
-    const int v1 = SPLIT ? min(nvec, v0 + cv) : nvec;
+    const int own = SPLIT ? static_cast<int>(blockIdx.y) : 0;
+    auto unit = [&](int i) { return buf_load16(xr, (threadIdx.x + static_cast<uint32_t>(i) * NT) * 16u); };
     uint4 v[VPT];
     uint32_t amax = 0u;
+    if (SPLIT && static_cast<int>(gridDim.y) > VPT) {
+        for (int i = 0; i < static_cast<int>(gridDim.y); ++i) amax = max(amax, abs_bits_max8(unit(i)));
+        v[0] = unit(own);
+    } else {
 #pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int idx = v0 + static_cast<int>(threadIdx.x) + i * NT;
-        v[i] = (idx < v1) ? xr[idx] : make_uint4(0u, 0u, 0u, 0u);
-        amax = max(amax, abs_bits_max8(v[i]));
-    }
-    if constexpr (SPLIT) {
-#pragma unroll 4
-        for (int idx = static_cast<int>(threadIdx.x); idx < nvec; idx += NT)
-            if (idx < v0 || idx >= v1) amax = max(amax, abs_bits_max8(xr[idx]));
+        for (int i = 0; i < VPT; ++i) v[i] = unit(i);
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) amax = max(amax, abs_bits_max8(v[i]));
+        if constexpr (SPLIT) {
+            uint4 w = v[0];
+#pragma unroll
+            for (int i = 1; i < VPT; ++i)
+                if (i == own) w = v[i];
+            v[0] = w;
+        }
     }
     amax = block_max<NT>(amax, red);
     const uint32_t sbits = scale_from_amax(amax);
     const RowScale q = row_scale(bf16_bits_to_f32(sbits));
-    const bool first = !SPLIT || blockIdx.y == 0;
+    const bool first = own == 0;
     if (threadIdx.x == 0 && first) ascale[row] = static_cast<uint16_t>(sbits);
     int8_t* qr = aq + row * lda;
-    // one uniform branch per row, not per element
-    auto emit = [&](auto fast) __attribute__((always_inline)) {
-        constexpr bool F = decltype(fast)::value;
 #pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int idx = v0 + static_cast<int>(threadIdx.x) + i * NT;
-            if (idx < v1) {
-                uint2 o;
-                o.x = quant2<F>(v[i].x, q) | (quant2<F>(v[i].y, q) << 16);
-                o.y = quant2<F>(v[i].z, q) | (quant2<F>(v[i].w, q) << 16);
-                *reinterpret_cast<uint2*>(qr + (PAD ? pad_dst(idx * 8, pm) : idx * 8)) = o;
-            }
-        }
-    };
-    if (q.fast) emit(std::true_type{});
-    else emit(std::false_type{});
+    for (int i = 0; i < (SPLIT ? 1 : VPT); ++i) {
+        const int idx = static_cast<int>(threadIdx.x) + (SPLIT ? own : i) * NT;
+        const uint2 o = quant_unit(v[i], q);
+        if (idx < nvec) *reinterpret_cast<uint2*>(qr + (PAD ? pad_dst(idx * 8, pm) : idx * 8)) = o;
+    }
     if constexpr (PAD) {
         if (first) zero_pads<8>(qr, K, pm);
     }
@@ -173,25 +173,31 @@ hipError_t launch_quant_act(const uint16_t* x, int64_t ldx, int8_t* a_q, int64_t
                          (reinterpret_cast<uintptr_t>(a_q) % 8 == 0);
     const int64_t nvec = K / 8;
     const int iK = static_cast<int>(K);
-    const int cv = static_cast<int>(nvec);
     // Rows of up to 8192 elements: 256 threads.  Longer rows of a small batch
-    // (M < 256, too few rows to fill the GPU): 1024-unit chunks, one 1024-
-    // thread workgroup each; longer rows otherwise: 1024 threads per row.
-    if (aligned && nvec > 4 * kThreads && M < 256) {
-        const int chunks = static_cast<int>((nvec + 1023) / 1024);
-        const dim3 g2(static_cast<unsigned>(M), static_cast<unsigned>(chunks));
-        if (pad) quant_act_vec_kernel<1, 1024, true, true><<<g2, dim3(1024), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm, 1024);
-        else quant_act_vec_kernel<1, 1024, false, true><<<g2, dim3(1024), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm, 1024);
+    // (M < 256, too few rows to fill the GPU) are split: over 512-thread workgroups
+    // of one 16-byte unit per thread up to 16 rows, 1024-thread ones past them
+    // (K = 27648, us: 16 rows 3.7 / 4.0, 64 rows 5.2 / 4.8, 200 rows 9.5 / 8.7).
+    // Longer rows otherwise: 1024 threads per row.
+    const bool vec = aligned && K < (int64_t{1} << 30);   // rows in 32-bit buffer offsets
+    if (vec && nvec > 4 * kThreads && M < 256) {
+        const int nt = M <= 16 ? 512 : 1024;
+        const dim3 g2(static_cast<unsigned>(M), static_cast<unsigned>((nvec + nt - 1) / nt));
+#define W4A8_QSPLIT(V, NT)                                                                                     \
+    if (pad) quant_act_vec_kernel<V, NT, true, true><<<g2, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm); \
+    else quant_act_vec_kernel<V, NT, false, true><<<g2, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm);
+        if (nt == 512) { W4A8_QSPLIT(8, 512) }
+        else { W4A8_QSPLIT(4, 1024) }
+#undef W4A8_QSPLIT
         return hipGetLastError();
     }
     int vpt = 0;
     const bool wide = nvec > 4 * kThreads;
     const int nt = wide ? 4 * kThreads : kThreads;
     for (int v : {1, 2, 4, 8})
-        if (vpt == 0 && aligned && nvec <= v * nt) vpt = v;
+        if (vpt == 0 && vec && nvec <= v * nt) vpt = v;
 #define W4A8_QVEC(V, NT)                                                                                      \
-    if (pad) quant_act_vec_kernel<V, NT, true, false><<<grid, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm, cv); \
-    else quant_act_vec_kernel<V, NT, false, false><<<grid, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm, cv);
+    if (pad) quant_act_vec_kernel<V, NT, true, false><<<grid, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm); \
+    else quant_act_vec_kernel<V, NT, false, false><<<grid, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm);
     if (vpt == 0) {
         quant_act_scalar_kernel<<<grid, block, 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pad, pm);
     } else if (!wide) {

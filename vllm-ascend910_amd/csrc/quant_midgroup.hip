@@ -62,20 +62,15 @@ __device__ __forceinline__ uint4 load8(const uint16_t* xr, int k0, int real, boo
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Eight codes -> four bytes of each plane (slot j in nibble j: even k low).
-template <bool FAST>
-__device__ __forceinline__ void pack8(const uint4& v, const RowScale& q, uint32_t& hw, uint32_t& lw, int& ksum) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-    hw = 0u;
-    lw = 0u;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const uint32_t u = w[j >> 1];
-        const int c = quant_code<FAST>(__uint_as_float((j & 1) ? (u & 0xffff0000u) : (u << 16)), q);
-        ksum += c;
-        hw |= (static_cast<uint32_t>(c >> 4) & 0xfu) << (4 * j);
-        lw |= ((static_cast<uint32_t>(c) & 0xfu) ^ 0x8u) << (4 * j);
-    }
+// Eight codes (one per byte) -> four bytes of each plane (slot j in nibble j: even k
+// low) and their sum.
+__device__ __forceinline__ void pack8(const uint2& c, uint32_t& hw, uint32_t& lw, int& ksum) {
+    // the nibbles of each byte pair side by side in bytes 0 and 2
+    auto pairs = [](uint32_t n) { return n | (n >> 4); };
+    hw = __builtin_amdgcn_perm(pairs((c.y >> 4) & 0x0f0f0f0fu), pairs((c.x >> 4) & 0x0f0f0f0fu), 0x06040200u);
+    lw = __builtin_amdgcn_perm(pairs(c.y & 0x0f0f0f0fu), pairs(c.x & 0x0f0f0f0fu), 0x06040200u) ^ 0x88888888u;
+    ksum = __builtin_amdgcn_sdot4(static_cast<int>(c.x), 0x01010101, ksum, false);
+    ksum = __builtin_amdgcn_sdot4(static_cast<int>(c.y), 0x01010101, ksum, false);
 }
 
 // kRowsMG rows per workgroup, their first loads all in flight together.
@@ -111,9 +106,7 @@ __global__ __launch_bounds__(kThreadsMG) void quant_midgroup_kernel(const MidQua
         amax[r] = abs_bits_max8(v0[r]);
         if (row0 + r < p.M)
             for (int c = tid + kThreadsMG; c < chunks; c += kThreadsMG) amax[r] = max(amax[r], abs_bits_max8(load8(src(r), 8 * c, real, vec)));
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1)
-            amax[r] = max(amax[r], static_cast<uint32_t>(__shfl_xor(static_cast<int>(amax[r]), off, 64)));
+        amax[r] = wave_max(amax[r]);
         if ((tid & 63) == 0) red_max[r][tid >> 6] = amax[r];
     }
     __syncthreads();
@@ -138,13 +131,11 @@ __global__ __launch_bounds__(kThreadsMG) void quant_midgroup_kernel(const MidQua
         for (int c = tid; c < chunks; c += kThreadsMG) {
             const uint4 v = c == tid ? v0[r] : (live ? load8(src(r), 8 * c, real, vec) : make_uint4(0u, 0u, 0u, 0u));
             uint32_t hw, lw;
-            if (q.fast) pack8<true>(v, q, hw, lw, ksum[r]);
-            else pack8<false>(v, q, hw, lw, ksum[r]);
+            pack8(quant_unit(v, q), hw, lw, ksum[r]);
             *reinterpret_cast<uint32_t*>(hrow + 4 * c) = hw;
             *reinterpret_cast<uint32_t*>(lrow + 4 * c) = lw;
         }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) ksum[r] += __shfl_xor(ksum[r], off, 64);
+        ksum[r] = wave_sum(ksum[r]);
         if ((tid & 63) == 0) red_sum[r][tid >> 6] = ksum[r];
     }
     __syncthreads();

@@ -17,8 +17,6 @@
 // (the updated residual stream) and h.  One workgroup per row, the row held in
 // registers (256 threads up to 8192 elements -- one 8-element unit per thread
 // for up to 64 rows -- and 1024 threads up to 65536).
-#include <type_traits>
-
 #include "common.h"
 #include "kgeom.h"
 #include "launch.h"
@@ -47,10 +45,8 @@ struct RmsParams {
     bool pad;
 };
 
-__device__ __forceinline__ float bf16r(float v) { return bf16_bits_to_f32(f32_to_bf16_bits(v)); }
-
 // Sum of the VPT per-unit partials v[i] of every thread, where thread t holds
-// unit t + i NT: unit-index bits 0-5 are the lane (xor shuffles, bit 0 first),
+// unit t + i NT: unit-index bits 0-5 are the lane (wave_sum's pairing, bit 0 first),
 // the next log2(NT / 64) bits the wave, the bits above the register index i
 // -- so pairing lanes, then waves, then registers, each in increasing bit
 // order, is the tree over the unit index, for every NT.
@@ -58,9 +54,7 @@ template <int VPT, int NT>
 __device__ __forceinline__ float block_sum_units(float (&v)[VPT], float* red) {
     constexpr int NW = NT / 64;
 #pragma unroll
-    for (int i = 0; i < VPT; ++i)
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) v[i] += __shfl_xor(v[i], off, 64);
+    for (int i = 0; i < VPT; ++i) v[i] = wave_sum(v[i]);
     if ((threadIdx.x & 63) == 0) {
 #pragma unroll
         for (int i = 0; i < VPT; ++i) red[i * NW + (threadIdx.x >> 6)] = v[i];
@@ -88,8 +82,7 @@ __device__ __forceinline__ float block_sum_units(float (&v)[VPT], float* red) {
 
 template <int NT>
 __device__ __forceinline__ uint32_t block_max_u(uint32_t v, uint32_t* red) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, 64)));
+    v = wave_max(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     uint32_t m = red[0];
@@ -107,39 +100,36 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     __shared__ uint32_t redu[NT / 64];
     const int64_t row = blockIdx.x;
     const int nvec = p.K >> 3;
-    const uint4* xr = reinterpret_cast<const uint4*>(p.x + row * p.ldx);
-    const uint4* rr = RES ? reinterpret_cast<const uint4*>(p.res + row * p.ldr) : nullptr;
-    const uint4* wr = reinterpret_cast<const uint4*>(p.w);
-
-    // the norm weight is requested with the row (it is used after the
-    // reduction, which would otherwise wait for a second memory round trip)
-    uint4 wv[VPT];
+    // Buffer loads (units past the row read zero), all requested before the first
+    // is used: the row, the residual, and the norm weight (used after the
+    // reduction, which would otherwise wait for a second memory round trip).
+    const uint32_t bytes = static_cast<uint32_t>(p.K) * 2u;
+    const auto xr = make_rsrc(p.x + row * p.ldx, bytes);
+    const auto rr = make_rsrc(RES ? p.res + row * p.ldr : p.x, RES ? bytes : 0u);
+    const auto wr = make_rsrc(p.w, bytes);
+    uint4 xv[VPT], rv[VPT], wv[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-        const int idx = static_cast<int>(threadIdx.x) + i * NT;
-        wv[i] = idx < nvec ? wr[idx] : make_uint4(0u, 0u, 0u, 0u);
+        const uint32_t o = (threadIdx.x + static_cast<uint32_t>(i * NT)) * 16u;
+        xv[i] = buf_load16(xr, o);
+        if constexpr (RES) rv[i] = buf_load16(rr, o);
     }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) wv[i] = buf_load16(wr, (threadIdx.x + static_cast<uint32_t>(i * NT)) * 16u);
     // s = bf16(x + r) kept as packed bf16 pairs; per-thread sum of squares
     uint4 v[VPT];
     float ss[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-        const int idx = static_cast<int>(threadIdx.x) + i * NT;
-        uint4 a = make_uint4(0u, 0u, 0u, 0u);
-        if (idx < nvec) {
-            a = xr[idx];
-            if constexpr (RES) {
-                const uint4 b = rr[idx];
-                uint32_t* pa = reinterpret_cast<uint32_t*>(&a);
-                const uint32_t* pb = reinterpret_cast<const uint32_t*>(&b);
+        uint4 a = xv[i];
+        if constexpr (RES) {
+            uint32_t* pa = reinterpret_cast<uint32_t*>(&a);
+            const uint32_t* pb = reinterpret_cast<const uint32_t*>(&rv[i]);
 #pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    const uint32_t lo = f32_to_bf16_bits(__uint_as_float(pa[d] << 16) + __uint_as_float(pb[d] << 16));
-                    const uint32_t hi = f32_to_bf16_bits(__uint_as_float(pa[d] & 0xffff0000u) +
-                                                         __uint_as_float(pb[d] & 0xffff0000u));
-                    pa[d] = lo | (hi << 16);
-                }
-            }
+            for (int d = 0; d < 4; ++d)
+                pa[d] = f32x2_to_bf16x2_bits(__uint_as_float(pa[d] << 16) + __uint_as_float(pb[d] << 16),
+                                             __uint_as_float(pa[d] & 0xffff0000u) +
+                                                 __uint_as_float(pb[d] & 0xffff0000u));
         }
         v[i] = a;
         const uint32_t* pa = reinterpret_cast<const uint32_t*>(&v[i]);
@@ -159,19 +149,19 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int idx = static_cast<int>(threadIdx.x) + i * NT;
-        if (idx >= nvec) continue;
-        if (p.sum_out) *reinterpret_cast<uint4*>(p.sum_out + row * p.lds + idx * 8) = v[i];
+        if (p.sum_out && idx < nvec) *reinterpret_cast<uint4*>(p.sum_out + row * p.lds + idx * 8) = v[i];
+        // (units past the row: zeros times a zero weight)
         uint32_t* pa = reinterpret_cast<uint32_t*>(&v[i]);
         const uint32_t* pw = reinterpret_cast<const uint32_t*>(&wv[i]);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            const float h0 = bf16r(bf16r(__uint_as_float(pa[d] << 16) * r) * __uint_as_float(pw[d] << 16));
-            const float h1 = bf16r(bf16r(__uint_as_float(pa[d] & 0xffff0000u) * r) *
-                                   __uint_as_float(pw[d] & 0xffff0000u));
-            pa[d] = (__float_as_uint(h0) >> 16) | (__float_as_uint(h1) & 0xffff0000u);
-            amax = max(amax, max(pa[d] & 0x7fffu, (pa[d] >> 16) & 0x7fffu));
+            const uint32_t n = f32x2_to_bf16x2_bits(__uint_as_float(pa[d] << 16) * r,
+                                                    __uint_as_float(pa[d] & 0xffff0000u) * r);
+            pa[d] = f32x2_to_bf16x2_bits(__uint_as_float(n << 16) * __uint_as_float(pw[d] << 16),
+                                         __uint_as_float(n & 0xffff0000u) * __uint_as_float(pw[d] & 0xffff0000u));
         }
-        if (p.h_out) *reinterpret_cast<uint4*>(p.h_out + row * p.ldh + idx * 8) = v[i];
+        amax = max(amax, abs_bits_max8(v[i]));
+        if (p.h_out && idx < nvec) *reinterpret_cast<uint4*>(p.h_out + row * p.ldh + idx * 8) = v[i];
     }
     amax = block_max_u<NT>(amax, redu);
     uint32_t sbits = f32_to_bf16_bits(bf16_bits_to_f32(amax) / 127.0f);
@@ -179,35 +169,18 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     const RowScale sc = row_scale(bf16_bits_to_f32(sbits));
     if (threadIdx.x == 0) p.a_scale[row] = static_cast<uint16_t>(sbits);
     int8_t* qr = p.a_q + row * p.lda;
-    // one uniform branch per row between the reciprocal and divide paths
-    auto emit = [&](auto fast) __attribute__((always_inline)) {
-        constexpr bool F = decltype(fast)::value;
 #pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int idx = static_cast<int>(threadIdx.x) + i * NT;
-            if (idx >= nvec) continue;
-            const uint32_t* pa = reinterpret_cast<const uint32_t*>(&v[i]);
-            uint2 o;
-            uint32_t wd[2] = {0u, 0u};
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const int q0 = quant_code<F>(__uint_as_float(pa[d] << 16), sc);
-                const int q1 = quant_code<F>(__uint_as_float(pa[d] & 0xffff0000u), sc);
-                wd[d >> 1] |= ((static_cast<uint32_t>(q0) & 0xffu) | ((static_cast<uint32_t>(q1) & 0xffu) << 8))
-                              << (16 * (d & 1));
-            }
-            o.x = wd[0];
-            o.y = wd[1];
-            int k0 = idx * 8;
-            if (p.pad) {
-                const int g = k0 / p.group;
-                k0 = g * p.stride + (k0 - g * p.group);
-            }
-            *reinterpret_cast<uint2*>(qr + k0) = o;
+    for (int i = 0; i < VPT; ++i) {
+        const int idx = static_cast<int>(threadIdx.x) + i * NT;
+        const uint2 o = quant_unit(v[i], sc);
+        if (idx >= nvec) continue;
+        int k0 = idx * 8;
+        if (p.pad) {
+            const int g = k0 / p.group;
+            k0 = g * p.stride + (k0 - g * p.group);
         }
-    };
-    if (sc.fast) emit(std::true_type{});
-    else emit(std::false_type{});
+        *reinterpret_cast<uint2*>(qr + k0) = o;
+    }
     if (p.pad) {
         // zero the padding slots (real lengths are multiples of 8 here)
         const int kp = static_cast<int>(geom::kpad(p.K, p.group));

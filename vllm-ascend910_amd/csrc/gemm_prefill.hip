@@ -90,7 +90,6 @@ struct PrefillParams {
     uint32_t a_bytes, w_bytes, s_bytes;
     bool vec_out;      // y 16-byte aligned with ldy % 8 == 0: 16-byte output stores
     int bm;            // tile rows: 128 or 64
-    bool cols;         // group stride 128 at 128 rows: 128 x 32 wave tiles (gemm_prefill_cols_kernel)
     int splits;        // gemm_prefill_cols_kernel: workgroups along K (blockIdx.y); > 1 writes fp32 sums to R
     float* R;          // splits > 1: fp32 sums before the token scale [splits, M, ldr]
     int64_t ldr;       // NB * 16
@@ -150,6 +149,38 @@ __device__ __forceinline__ void store_tile(const PrefillParams& p, const uint16_
 #pragma unroll
             for (int q = 0; q < 8; ++q)
                 if (col + q < ncols) y[q] = static_cast<uint16_t>(w[q >> 1] >> (16 * (q & 1)));
+        }
+    }
+}
+
+// The same for a tile of kBN / 2 gate columns and their kBN / 2 up columns side by
+// side: 8 outputs silu(g) * u per thread and step.
+template <int BM, int THREADS, int OS>
+__device__ __forceinline__ void store_tile_swiglu(const PrefillParams& p, const uint16_t* lo, const uint16_t* hi,
+                                                  int m0, int n0, int tid) {
+    constexpr int OC = kBN / 2, CPR = OC / 8;
+#pragma unroll
+    for (int k = 0; k < BM * CPR / THREADS; ++k) {
+        const int c = tid + k * THREADS;
+        const int r = c / CPR, c8 = (c % CPR) * 8;
+        const int row = m0 + r, col = n0 + c8;
+        if (row >= p.M || col >= p.half_n) continue;
+        const uint16_t* src = (r < BM / 2 ? lo : hi) + (r % (BM / 2)) * OS + c8;
+        const uint4 gv = *reinterpret_cast<const uint4*>(src);
+        const uint4 uv = *reinterpret_cast<const uint4*>(src + OC);
+        const uint32_t g[4] = {gv.x, gv.y, gv.z, gv.w}, u[4] = {uv.x, uv.y, uv.z, uv.w};
+        uint32_t w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            w[q] = swiglu_bf16_bits(__uint_as_float(g[q] << 16), __uint_as_float(u[q] << 16)) |
+                   (swiglu_bf16_bits(__uint_as_float(g[q] & 0xffff0000u), __uint_as_float(u[q] & 0xffff0000u)) << 16);
+        uint16_t* y = p.Y + static_cast<int64_t>(row) * p.ldy + col;
+        if (p.vec_out && col + 8 <= p.half_n) {
+            *reinterpret_cast<uint4*>(y) = make_uint4(w[0], w[1], w[2], w[3]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (col + q < p.half_n) y[q] = static_cast<uint16_t>(w[q >> 1] >> (16 * (q & 1)));
         }
     }
 }
@@ -681,7 +712,7 @@ __global__ __launch_bounds__(threads_for<BM>(), 2) void gemm_prefill_kernel(cons
 
 constexpr int kDW = 2;   // weight prefetch depth in K steps
 
-// Group stride 128 without the partial dump or the SwiGLU pairs: the same
+// Group stride 128 without the partial dump: the same
 // BM x 128 tile (BM = 128 or 64) and K step, but each of the four waves owns
 // all BM rows and one 32-column block (instead of 64 x 64 per wave; at 64
 // rows, four waves per tile instead of two, three workgroups per CU).  Every weight is then loaded and
@@ -692,7 +723,12 @@ constexpr int kDW = 2;   // weight prefetch depth in K steps
 // rb's fold runs during row block rb + 1's MFMAs (row block 3's during the next
 // step's row block 0), one MFMA to eight fold instructions.  Each output's
 // arithmetic is the 64 x 64 kernel's: outputs are bit-identical.
-template <bool SBF16, int BM>
+// SWIGLU: the tile's 128 columns are 64 gate columns (waves 0 and 1) and the
+// matching 64 up columns (waves 2 and 3); the bf16 gate and up values meet in the
+// output tile in LDS, and silu(g) * u is formed on the way out.  Every column
+// accumulates as in the plain GEMM (gate_up with SwiGLU against the 64 x 64 waves:
+// 256 rows 119 -> 104 us, 1024 375 -> 360, 4096 1398 -> 1365).
+template <bool SBF16, int BM, bool SWIGLU>
 __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kernel(const PrefillParams p) {
     constexpr int kBM = BM, kThreads = 256;
     constexpr int RB = BM / 32;                  // 32-row blocks per wave
@@ -712,7 +748,7 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kerne
     int tile_m, tile_n;
     tile_of(p, tile_m, tile_n);
     const int m0 = tile_m * kBM;
-    const int n0 = tile_n * kBN;
+    const int n0 = tile_n * (SWIGLU ? kBN / 2 : kBN);
     const int c32 = lane & 31;
     const int hh = lane >> 5;
     // This workgroup's K steps [ka, ka + nk): the KT steps split evenly over
@@ -732,7 +768,7 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kerne
     if (tid < kBM && m0 + tid < p.M) ts_bits = p.a_scale[m0 + tid];
 
     // weights: this lane's two 16-byte chunks per step of the wave's block
-    const int col = n0 + wave * 32 + c32;
+    const int col = SWIGLU ? n0 + (wave & 1) * 32 + c32 + (wave >> 1) * p.half_n : n0 + wave * 32 + c32;
     const uint32_t tile0 = static_cast<uint32_t>(col >> 4) * static_cast<uint32_t>(p.KT) * 1024u;
     const uint32_t woff0 = tile0 + static_cast<uint32_t>((col & 15) + 16 * hh) * 16u;        // slabs 0, 2
     const uint32_t woff1 = tile0 + static_cast<uint32_t>((col & 15) + 16 * (2 + hh)) * 16u;  // slabs 1, 3
@@ -892,8 +928,10 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kerne
             }
         }
     __syncthreads();
-    store_tile<kBM, kThreads, OC, OS>(p, reinterpret_cast<const uint16_t*>(la0), reinterpret_cast<const uint16_t*>(la1),
-                                      m0, n0, p.N, tid);
+    const auto* lo = reinterpret_cast<const uint16_t*>(la0);
+    const auto* hi = reinterpret_cast<const uint16_t*>(la1);
+    if constexpr (SWIGLU) store_tile_swiglu<kBM, kThreads, OS>(p, lo, hi, m0, n0, tid);
+    else store_tile<kBM, kThreads, OC, OS>(p, lo, hi, m0, n0, p.N, tid);
 }
 
 // The reference's mid-group activation planes rebuilt for the compat variant
@@ -945,17 +983,17 @@ hipError_t launch_g(const PrefillParams& p, hipStream_t stream) {
     // The partial dump keeps 128-row tiles (the compiler fails on the 64-row
     // dump variants); each output element's arithmetic does not depend on the
     // tile height, so its outputs equal the 64-row kernel's bit for bit.
-    if constexpr (GMODE == 1 && !DUMP && !SWIGLU) {
-        if (p.cols) {
-            if (p.bm == 128) gemm_prefill_cols_kernel<SBF16, 128><<<grid, dim3(256), 0, stream>>>(p);
-            else gemm_prefill_cols_kernel<SBF16, 64><<<grid, dim3(256), 0, stream>>>(p);
-            return hipGetLastError();
-        }
+    if constexpr (GMODE == 1 && !DUMP) {
+        if (p.bm == 128) gemm_prefill_cols_kernel<SBF16, 128, SWIGLU><<<grid, dim3(256), 0, stream>>>(p);
+        else gemm_prefill_cols_kernel<SBF16, 64, SWIGLU><<<grid, dim3(256), 0, stream>>>(p);
+    } else if constexpr (DUMP) {
+        gemm_prefill_kernel<GMODE, kDW, SBF16, true, SWIGLU, 128><<<grid, dim3(threads_for<128>()), 0, stream>>>(p);
+    } else {
+        if (p.bm == 64)
+            gemm_prefill_kernel<GMODE, kDW, SBF16, false, SWIGLU, 64><<<grid, dim3(threads_for<64>()), 0, stream>>>(p);
+        else
+            gemm_prefill_kernel<GMODE, kDW, SBF16, false, SWIGLU, 128><<<grid, dim3(threads_for<128>()), 0, stream>>>(p);
     }
-    if (p.bm == 64 && !DUMP)
-        gemm_prefill_kernel<GMODE, kDW, SBF16, false, SWIGLU, 64><<<grid, dim3(threads_for<64>()), 0, stream>>>(p);
-    else
-        gemm_prefill_kernel<GMODE, kDW, SBF16, DUMP, SWIGLU, 128><<<grid, dim3(threads_for<128>()), 0, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -968,12 +1006,6 @@ hipError_t launch(const PrefillParams& p, hipStream_t stream) {
 }
 
 }  // namespace
-
-// The 128 x 32 wave tiles for group stride 128 (defined 0 only for
-// side-by-side measurements of the 64 x 64 kernel).
-#ifndef W4A8_PREFILL_COLS
-#define W4A8_PREFILL_COLS 1
-#endif
 
 int64_t prefill_workspace_bytes(int64_t, int64_t, int64_t, int64_t) { return 0; }
 
@@ -1117,7 +1149,7 @@ hipError_t launch_gemm_midgroup_prefill(const MidgroupArgs& a, void* ws, int64_t
 int prefill_tile_rows(int64_t M, int64_t N, int64_t group, bool swiglu) {
     const int64_t tn = swiglu ? geom::ceil_div(N / 2, kBN / 2) : geom::ceil_div(N, kBN);
     const int64_t tiles = geom::ceil_div(M, int64_t{128}) * tn, cus = device_cu_count();
-    if (W4A8_PREFILL_COLS && !swiglu && geom::group_stride(group) == 128) {
+    if (geom::group_stride(group) == 128) {
         // The four-wave tiles of gemm_prefill_cols_kernel (64-row tiles run
         // three workgroups per CU, 128-row tiles two).  64 rows up to 1.5
         // tiles of 128 rows per CU and between 2 and 4 per CU; 128 rows where
@@ -1128,7 +1160,7 @@ int prefill_tile_rows(int64_t M, int64_t N, int64_t group, bool swiglu) {
         // 179 / 198; gate_up M=256 86 / 88, M=512 167 / 156.
         return (tiles * 2 <= cus * 3 || (tiles > 2 * cus && tiles <= 4 * cus)) ? 64 : 128;
     }
-    // The 64 x 64 wave tiles (other group strides, SwiGLU): 64-row tiles
+    // The 64 x 64 wave tiles (other group strides): 64-row tiles
     // (twice as many, up to four workgroups per CU) where the 128-row ones
     // would leave CUs idle or unevenly loaded: at most one for every second
     // CU, or between one and two per CU.  Measured on MI355X (QwQ-32B shapes,
@@ -1182,13 +1214,12 @@ hipError_t launch_gemm_prefill_split(const GemmArgs& a, int splits, hipStream_t 
     p.w_bytes = static_cast<uint32_t>(geom::col_blocks(a.N) * geom::k_tiles(a.K, a.group) * geom::kTileBytes);
     p.s_bytes = static_cast<uint32_t>(geom::col_blocks(a.N) * geom::num_groups(a.K, a.group) * 16 * 2);
     p.vec_out = (reinterpret_cast<uintptr_t>(a.y) % 16 == 0) && (a.ldy % 8 == 0);
-    p.cols = true;
     p.splits = need > 0 ? static_cast<int>(std::min<int64_t>(splits, p.KT)) : 1;
     p.R = static_cast<float*>(a.workspace);
     p.ldr = static_cast<int64_t>(p.NB) * 16;
     const dim3 grid(static_cast<unsigned>(p.tiles_n), static_cast<unsigned>(p.splits));
-    if (a.scale_bf16) gemm_prefill_cols_kernel<true, 64><<<grid, dim3(256), 0, stream>>>(p);
-    else gemm_prefill_cols_kernel<false, 64><<<grid, dim3(256), 0, stream>>>(p);
+    if (a.scale_bf16) gemm_prefill_cols_kernel<true, 64, false><<<grid, dim3(256), 0, stream>>>(p);
+    else gemm_prefill_cols_kernel<false, 64, false><<<grid, dim3(256), 0, stream>>>(p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.splits == 1) return e;
     return launch_split_reduce(p.R, p.ldr, p.a_scale, p.Y, p.ldy, p.M, p.N, p.splits, false, a.scale_bf16, p.S,
@@ -1227,7 +1258,6 @@ hipError_t launch_gemm_prefill_bm(const GemmArgs& a, int bm, hipStream_t stream)
     p.w_bytes = static_cast<uint32_t>(geom::col_blocks(a.N) * geom::k_tiles(a.K, a.group) * geom::kTileBytes);
     p.s_bytes = static_cast<uint32_t>(geom::col_blocks(a.N) * geom::num_groups(a.K, a.group) * 16 * 2);
     p.vec_out = (reinterpret_cast<uintptr_t>(a.y) % 16 == 0) && (a.ldy % 8 == 0);
-    p.cols = W4A8_PREFILL_COLS != 0;
     p.splits = 1;
     if (a.swiglu) return a.scale_bf16 ? launch<true, false, true>(p, stream) : launch<false, false, true>(p, stream);
     const bool dump = a.partials != nullptr;

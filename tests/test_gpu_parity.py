@@ -1053,6 +1053,15 @@ def test_gemm_swiglu(pkg, dev, M, I, K, G, sd):
     assert np.mean(got == exp) > 0.99
 
 
+@pytest.mark.parametrize("M,I,K,G,sd", [
+    (1000, 3856, 384, 128, "bf16"),  # 128-row tiles of 64 gate + 64 up columns, I not a multiple of 64
+    (65, 48, 300, 128, "f16"),       # one 64-row tile past its rows and columns, ragged K
+    (129, 64, 128, 128, "bf16"),     # one K step
+])
+def test_gemm_swiglu_prefill_tiles(pkg, dev, M, I, K, G, sd):
+    test_gemm_swiglu(pkg, dev, M, I, K, G, sd)
+
+
 @pytest.mark.parametrize("M,I,K,G,sd", [(m, max(16, n // 32 * 16), k, g, sd)
                                         for m, n, k, g, sd in random_shapes(4242, 16 * RANDOM_SCALE)])
 def test_gemm_swiglu_random_shapes(pkg, dev, M, I, K, G, sd):

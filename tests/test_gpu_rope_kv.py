@@ -123,6 +123,41 @@ def test_rope_kv_strided_k_cache(pkg, dev):
     assert bits_equal(k_view, kc_ref) and bits_equal(vc, vc_ref)
 
 
+@pytest.mark.parametrize("B,T,H,KVH,D,L,p0,with_bias", [
+    (8, 16, 40, 8, 128, 64, 3, True),      # the fewest tokens of the prefill kernel
+    (2, 65, 4, 2, 64, 70, 5, False),       # a v tile and one token, an odd offset
+    (2, 150, 10, 2, 128, 192, 42, True),   # up to the last cache position
+    (2, 70, 6, 3, 96, 90, 30, True),       # ten tokens past the cache end, D = 96
+    (4, 33, 4, 2, 64, 64, -3, False),      # three tokens before position 0
+])
+def test_rope_kv_prefill_layout(pkg, dev, B, T, H, KVH, D, L, p0, with_bias):
+    """The decoder's cache layouts (K rows contiguous, V transposed) against the torch path
+    and against the same call on caches of the other layouts: the same bits."""
+    say(f"rope_kv prefill layout B={B} T={T} H={H} KVH={KVH} D={D} L={L} p0={p0} bias={with_bias}")
+    qkv, kc, vc = make(B, T, H, KVH, D, L, dev, seed=B * 100 + T)
+    cos, sin = tables(L, D, dev)
+    bias = None
+    if with_bias:
+        g = torch.Generator(device=dev).manual_seed(5)
+        bias = ((torch.rand(((H + 2 * KVH) * D,), device=dev, generator=g) - 0.5) * 0.2).to(torch.bfloat16)
+    pos = torch.tensor([p0], device=dev)
+    lc = -(-L // 64) * 64
+    k_store = torch.zeros((B, KVH, lc, D), dtype=torch.bfloat16, device=dev)
+    vt_store = torch.zeros((B, KVH, D, lc), dtype=torch.bfloat16, device=dev)
+    k_view, v_view = k_store[:, :, :L].transpose(2, 3), vt_store[..., :L].transpose(2, 3)
+    k_view.copy_(kc)
+    v_view.copy_(vc)
+    q = torch.ops.npu.w4a8_rope_kv(qkv, cos, sin, pos, k_view, v_view, H, KVH, bias)
+    kc2, vc2 = kc.clone(), vc.clone()
+    q2 = torch.ops.npu.w4a8_rope_kv(qkv, cos, sin, pos, kc2, vc2, H, KVH, bias)
+    torch.cuda.synchronize()
+    assert bits_equal(q, q2) and bits_equal(k_view, kc2) and bits_equal(v_view, vc2)
+    assert not k_store[:, :, L:].any() and not vt_store[..., L:].any()
+    t0, t1 = max(0, -p0), min(T, L - p0)                  # tokens inside the cache
+    q_ref, kc_ref, vc_ref = reference(qkv[:, t0:t1], cos, sin, p0 + t0, kc, vc, H, KVH, bias)
+    assert bits_equal(q[:, t0:t1], q_ref) and bits_equal(k_view, kc_ref) and bits_equal(v_view, vc_ref)
+
+
 def test_rope_kv_graph_replays_follow_the_position(pkg, dev):
     """Captured once; each replay reads the position from the device and the step advances it."""
     B, H, KVH, D, L = 2, 40, 8, 128, 32

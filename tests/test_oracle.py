@@ -331,6 +331,7 @@ def test_gemm_fp32_equals_reference_torch_loop():
     assert np.array_equal(ow.gemm_fp32(q, sb, w, ws, G), acc.numpy())
 
 
+@needs_ref
 def test_gemm_bf16_matches_reference_cpp():
     for seed, (M, N, K, G) in enumerate(((8, 64, 512, 128), (16, 128, 5120 // 4, 256), (4, 32, 1024, 64))):
         xb, w, wsb = _gemm_case(seed + 10, M, N, K, G)

@@ -1,0 +1,96 @@
+"""The C++ torch kernels (csrc/torch_ops.cpp): what is registered, the inputs they
+accept and refuse, and calls from several threads."""
+from __future__ import annotations
+
+import threading
+
+import pytest
+import torch
+
+OPS = ["w4a8_quant_pertoken", "w4a8_gemm", "w4a8_gemm_swiglu", "w4a8_linear", "w4a8_rmsnorm_quant", "w4a8_rope_kv",
+       "w4a8_attention", "w4a8_attention_rope", "midgroup_quant_a", "midgroup_w4a8_gemm", "midgroup_w4a8_gemm_tiled"]
+
+
+def test_native_ops_are_registered(pkg):
+    assert pkg._abi.TORCH_LIB_PATH.exists(), "csrc/torch_ops.cpp is not built"
+    for op in OPS:
+        assert torch._C._dispatch_has_kernel_for_dispatch_key(f"npu::{op}", "CUDA"), op
+        assert not torch._C._dispatch_has_kernel_for_dispatch_key(f"npu::{op}", "CPU"), op
+
+
+def _weight(dev, N, K, G, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    w_q = torch.randint(-128, 128, (N, K // 2), dtype=torch.int8, device=dev, generator=g)
+    ws = (torch.rand((K // G, N), device=dev, generator=g) * 0.018 + 0.002).to(torch.bfloat16)
+    return torch.ops.npu.w4a8_repack(w_q, ws, K, G)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 5, 70])
+def test_strided_inputs(pkg, dev, M):
+    """Row-strided, column-strided and 3-D inputs give the contiguous input's bits."""
+    N, K, G = 256, 1024, 128
+    w, s = _weight(dev, N, K, G, 3)
+    wide = torch.randn((M, 2 * K), device=dev).to(torch.bfloat16)
+    x = wide[:, :K].contiguous()
+    want = torch.ops.npu.w4a8_linear(x, w, s, N, K, G)
+    assert torch.equal(torch.ops.npu.w4a8_linear(wide[:, :K], w, s, N, K, G), want)
+    assert torch.equal(torch.ops.npu.w4a8_linear(x.t().contiguous().t(), w, s, N, K, G), want)
+    a_q, a_s = torch.ops.npu.w4a8_quant_pertoken(x)
+    wide_q = torch.zeros((M, K + 16), dtype=torch.int8, device=dev)
+    wide_q[:, :K] = a_q
+    odd_q = torch.zeros((M, K + 3), dtype=torch.int8, device=dev)   # rows not a multiple of 16 bytes apart
+    odd_q[:, :K] = a_q
+    # (a single row counts as contiguous whatever its stride, so its odd stride is refused)
+    for q in (a_q, wide_q[:, :K]) + ((odd_q[:, :K],) if M > 1 else ()):
+        assert torch.equal(torch.ops.npu.w4a8_gemm(q, a_s, w, s, N, K, G), want)
+    assert torch.equal(pkg.linear(x.view(1, M, K), w, s, N, G), want.view(1, M, N))
+    assert torch.equal(pkg.linear(x.float(), w, s, N, G), want)
+    assert torch.ops.npu.w4a8_linear(x[:0], w, s, N, K, G).shape == (0, N)
+
+
+@pytest.mark.gpu
+def test_bad_inputs_raise(pkg, dev):
+    N, K, G = 256, 1024, 128
+    w, s = _weight(dev, N, K, G, 4)
+    x = torch.randn((2, K), device=dev).to(torch.bfloat16)
+    for bad in (lambda: torch.ops.npu.w4a8_linear(x.float(), w, s, N, K, G),
+                lambda: torch.ops.npu.w4a8_linear(x[:, :512], w, s, N, K, G),
+                lambda: torch.ops.npu.w4a8_linear(x, w[:-1], s, N, K, G),
+                lambda: torch.ops.npu.w4a8_linear(x, w, s.float(), N, K, G),
+                lambda: torch.ops.npu.w4a8_linear(x, w, s, N, K, 0),
+                lambda: torch.ops.npu.w4a8_linear(x, w, s, -N, K, G),
+                lambda: torch.ops.npu.w4a8_quant_pertoken(x[0]),
+                lambda: torch.ops.npu.w4a8_quant_pertoken(x, -1),
+                lambda: torch.ops.npu.midgroup_quant_a(x, 0)):
+        with pytest.raises(RuntimeError):
+            bad()
+
+
+@pytest.mark.gpu
+def test_threads_with_their_own_streams(pkg, dev):
+    """Four threads, a stream each, calling a linear whose GEMM splits K (workspace per
+    stream) and one whose does not: every result is the single-threaded one."""
+    shapes = [(24, 1000 // 16 * 16, 16384, 128), (3, 512, 1024, 128)]
+    work = []
+    for i, (M, N, K, G) in enumerate(shapes):
+        w, s = _weight(dev, N, K, G, 10 + i)
+        x = torch.randn((M, K), device=dev).to(torch.bfloat16)
+        work.append((x, w, s, N, K, G, torch.ops.npu.w4a8_linear(x, w, s, N, K, G)))
+    torch.cuda.synchronize()
+    bad = []
+
+    def run(t):
+        with torch.cuda.stream(torch.cuda.Stream(device=dev)):
+            for i in range(20):
+                x, w, s, N, K, G, want = work[(i + t) % len(work)]
+                y = torch.ops.npu.w4a8_linear(x, w, s, N, K, G)
+                if not torch.equal(y, want):
+                    bad.append((t, i))
+
+    ts = [threading.Thread(target=run, args=(t,)) for t in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad

@@ -15,6 +15,7 @@ from pathlib import Path
 
 _HERE = Path(__file__).resolve().parent
 LIB_PATH = _HERE / "_lib" / "libw4a8_amd.so"
+TORCH_LIB_PATH = _HERE / "_lib" / "w4a8_torch.so"   # csrc/torch_ops.cpp
 ABI_VERSION = 10
 
 W4A8_DT_F16 = 0

@@ -22,18 +22,24 @@ from . import ops  # noqa: F401  (registers torch.ops.npu.*)
 from .packing import quantize_weight
 
 
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    """x as contiguous bf16 rows [M, K]; an activation that already is one passes through."""
+    if x.dim() == 2 and x.dtype is torch.bfloat16 and x.is_contiguous():
+        return x
+    return x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
+
+
 def linear(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor, N: int, group: int,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x @ W.T with per-token int8 activations and per-group int4 weights.
 
     The reference's ``w4a8_ops.linear`` (npu_ops/python/w4a8_ops.py:243-252).
     """
-    lead, K = x.shape[:-1], x.shape[-1]
-    x2 = x.reshape(-1, K).to(torch.bfloat16).contiguous()
-    y = torch.ops.npu.w4a8_linear(x2, w_tiles, s_tiles, N, K, group)
+    K = x.shape[-1]
+    y = torch.ops.npu.w4a8_linear(_rows(x), w_tiles, s_tiles, N, K, group)
     if bias is not None:
         y = y + bias
-    return y.reshape(*lead, N)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
 
 
 def linear_swiglu(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor, N: int, group: int
@@ -43,11 +49,10 @@ def linear_swiglu(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor,
     Equals ``g, u = linear(x, ...).split(N // 2, -1); F.silu(g) * u`` in bf16, the
     reference decoder layer's MLP activation (npu_ops/python/bench_decode_layer.py:78-81).
     """
-    lead, K = x.shape[:-1], x.shape[-1]
-    x2 = x.reshape(-1, K).to(torch.bfloat16).contiguous()
-    a_q, a_scale = torch.ops.npu.w4a8_quant_pertoken(x2, group)
+    K = x.shape[-1]
+    a_q, a_scale = torch.ops.npu.w4a8_quant_pertoken(_rows(x), group)
     y = torch.ops.npu.w4a8_gemm_swiglu(a_q, a_scale, w_tiles, s_tiles, N, K, group)
-    return y.reshape(*lead, N // 2)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N // 2)
 
 
 class W4A8Linear(nn.Module):
@@ -112,12 +117,11 @@ def midgroup_linear(x: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, wk: tor
     The reference's ``w4a8_ops.linear`` (npu_ops/python/w4a8_ops.py:243-252): quant_a pads the
     rows to TILE_M, so y has >= x's rows and is sliced before reshaping.
     """
-    lead, K = x.shape[:-1], x.shape[-1]
-    x2 = x.reshape(-1, K).to(torch.bfloat16).contiguous()
+    K, x2 = x.shape[-1], _rows(x)
     a_hi, a_lo, a_scale, a_ksum = torch.ops.npu.midgroup_quant_a(x2, group)
     # only the real rows (the reference slices them from the padded product)
     y = torch.ops.npu.midgroup_w4a8_gemm(a_hi, a_lo, a_scale, a_ksum, wq, ws, wk, wz, K, group, x2.shape[0])
-    return y.reshape(*lead, y.shape[-1])
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], y.shape[-1])
 
 
 class MidGroupW4A8Linear(nn.Module):
@@ -172,8 +176,7 @@ class MidGroupW4A8Linear(nn.Module):
         if self._gn is None:
             raise RuntimeError("MidGroupW4A8Linear: call process_weights_after_loading() after loading weights")
         ws, wk, wz = self._gn
-        lead, k = x.shape[:-1], x.shape[-1]
-        x2 = x.reshape(-1, k).to(torch.bfloat16).contiguous()
+        k, x2 = x.shape[-1], _rows(x)
         rows = x2.shape[0]
         a_hi, a_lo, a_scale, a_ksum = torch.ops.npu.midgroup_quant_a(x2, self.group)
         if self._tiles is not None and self._tiles.device == x2.device:
@@ -184,4 +187,4 @@ class MidGroupW4A8Linear(nn.Module):
                                                  self.group, rows)
         if self.bias is not None:
             y = y + self.bias
-        return y.reshape(*lead, self.out_features)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)

@@ -294,17 +294,16 @@ class W4A8Decoder:
                     o[b:b + 1] = self._attend(qg[b:b + 1].contiguous(), kc[b:b + 1], vc[b:b + 1], bias)
             out = o.view(B, c.kv_heads, G, S, c.head_dim).permute(0, 3, 1, 2, 4).reshape(B * S, c.heads * c.head_dim)
             x, delta = self._mlp_and_next(L, x, out)
-        last = (x + delta).view(B, S, c.hidden)[:, -1]
-        return self._logits_argmax(last)
+        return self._logits_argmax(x.view(B, S, c.hidden)[:, -1], delta.view(B, S, c.hidden)[:, -1])
 
-    def _logits(self, x_last: torch.Tensor) -> torch.Tensor:
-        c = self.cfg
-        v = x_last.float()
-        h = (v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + c.rms_eps)).to(torch.bfloat16) * self.final_norm
+    def _logits(self, x_last: torch.Tensor, delta: torch.Tensor) -> torch.Tensor:
+        """Final norm of x_last + delta (the residual add and both bf16 roundings of the
+        layers' norms, one launch where the elementwise form took nine) and the lm_head."""
+        _, _, _, h = torch.ops.npu.w4a8_rmsnorm_quant(x_last, self.final_norm, self.cfg.rms_eps, delta, 0, True)
         return torch.nn.functional.linear(h, self.lm_head)
 
-    def _logits_argmax(self, x_last: torch.Tensor) -> torch.Tensor:
-        logits = self._logits(x_last)
+    def _logits_argmax(self, x_last: torch.Tensor, delta: torch.Tensor) -> torch.Tensor:
+        logits = self._logits(x_last, delta)
         self.last_logits = logits
         return logits.argmax(dim=-1)
 
@@ -337,7 +336,7 @@ class W4A8Decoder:
             else:
                 o = self._attend(qg, self.k_cache[li], self.v_cache[li], bias)      # [B, KVH, G, D]
             x, delta = self._mlp_and_next(L, x, o.reshape(B, c.heads * c.head_dim))
-        self.tokens.copy_(self._logits_argmax(x + delta))
+        self.tokens.copy_(self._logits_argmax(x, delta))
         self.pos.add_(1)
 
     @torch.no_grad()

@@ -215,6 +215,16 @@ int w4a8_linear(const void* x, int64_t ldx, const void* w_tiles, const void* s_t
                 int64_t K, int64_t group, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * w4a8_linear with a bias (bf16 [N], 2-byte aligned, or NULL) added to the bf16
+ * outputs in the GEMM's epilogue: y = bf16(bf16(x @ W.T) + bias), the bits of a
+ * bf16 tensor add after w4a8_linear (the reference's apply,
+ * npu_ops/python/midgroup_quant.py:163-177).
+ */
+int w4a8_linear_bias(const void* x, int64_t ldx, const void* w_tiles, const void* s_tiles, int scale_dtype,
+                     const void* bias, void* y, int64_t ldy, void* a_q, int64_t lda, void* a_scale, int64_t M,
+                     int64_t N, int64_t K, int64_t group, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * 1 when w4a8_linear with these arguments runs as one fused launch, 0 when it
  * runs the quant and GEMM kernels (no counterpart in the reference: a query
  * for tests and schedulers; x is only inspected for alignment).

@@ -50,6 +50,64 @@ def test_strided_inputs(pkg, dev, M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,G", [
+    (1, 5120, 1024, 128),      # fused single row, staged decode plans
+    (5, 1000, 1024, 128),      # N off the 16-column tile
+    (16, 256, 1024, 64),
+    (40, 1000, 2048, 256),     # row groups
+    (12, 32800, 256, 128),     # wide kernel
+    (20, 1000, 16384, 128),    # wide kernel, K split: added by the reduce
+    (50, 1000, 16384, 128),    # split prefill tile
+    (12, 512, 16384, 16384),   # one group, int32 sums in the reduce
+    (70, 1000, 512, 128),      # 64-row prefill tiles, a ragged last column tile
+    (600, 7000, 256, 128),     # 128-row prefill tiles
+    (130, 1000, 1024, 64),     # 64 x 64 wave tiles
+])
+def test_linear_bias(pkg, dev, M, N, K, G):
+    """The epilogue's bias on every plan: the bits of the bf16 add after the linear."""
+    w, s = _weight(dev, N, K, G, M + N)
+    x = torch.randn((M, K), device=dev).to(torch.bfloat16)
+    bias = torch.randn((N,), device=dev).to(torch.bfloat16)
+    y = torch.ops.npu.w4a8_linear(x, w, s, N, K, G)
+    assert torch.equal(torch.ops.npu.w4a8_linear(x, w, s, N, K, G, bias), y + bias)
+    assert torch.equal(pkg.linear(x, w, s, N, G, bias), y + bias)
+
+
+@pytest.mark.gpu
+def test_linear_bias_left_to_torch(pkg, dev):
+    """Biases the epilogue does not take keep torch's own add: dtype promotion,
+    broadcasting, autograd and forward-mode derivatives."""
+    M, N, K, G = 3, 256, 512, 128
+    w, s = _weight(dev, N, K, G, 9)
+    x = torch.randn((M, K), device=dev).to(torch.bfloat16)
+    y = torch.ops.npu.w4a8_linear(x, w, s, N, K, G)
+    f32 = torch.randn((N,), device=dev)
+    assert pkg.linear(x, w, s, N, G, f32).dtype == torch.float32
+    col = torch.randn((M, 1), device=dev).to(torch.bfloat16)
+    assert torch.equal(pkg.linear(x, w, s, N, G, col), y + col)
+    b = f32.to(torch.bfloat16).requires_grad_()
+    pkg.linear(x, w, s, N, G, b).sum().backward()
+    assert b.grad is not None
+    with torch.no_grad():
+        assert torch.equal(pkg.linear(x, w, s, N, G, b), y + b)
+    import torch.autograd.forward_ad as fwd
+    with fwd.dual_level():
+        dual = fwd.make_dual(b.detach(), torch.ones_like(b))
+        assert torch.equal(fwd.unpack_dual(pkg.linear(x, w, s, N, G, dual)).tangent, torch.ones_like(y))
+    b2 = torch.stack([b.detach(), -b.detach()])
+    assert torch.equal(torch.func.vmap(lambda t: pkg.linear(x, w, s, N, G, t))(b2), y + b2[:, None])
+    assert torch.equal(torch.func.grad(lambda t: pkg.linear(x, w, s, N, G, t).sum())(b.detach()),
+                       torch.full_like(f32, M, dtype=torch.bfloat16))
+    with pytest.raises(RuntimeError):
+        torch.ops.npu.w4a8_linear(x, w, s, N, K, G, f32)
+    # read by the epilogue: a strided view, an odd offset, infinities and NaN
+    special = f32.to(torch.bfloat16)
+    special[:3] = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    for v in (torch.stack([special, special], 1)[:, 1], torch.cat([special[:1], special])[1:]):
+        torch.testing.assert_close(torch.ops.npu.w4a8_linear(x, w, s, N, K, G, v), y + v, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.gpu
 def test_bad_inputs_raise(pkg, dev):
     N, K, G = 256, 1024, 128
     w, s = _weight(dev, N, K, G, 4)

@@ -39,6 +39,8 @@ SIGNATURES = {
     "w4a8_gemm_noalloc": (_I, [_VP, _I64, _VP, _VP, _VP, _I, _VP, _I64, _I64, _I64, _I64, _I64, _VP]),
     "w4a8_gemm_swiglu": (_I, [_VP, _I64, _VP, _VP, _VP, _I, _VP, _I64, _I64, _I64, _I64, _I64, _VP, _I64, _VP]),
     "w4a8_linear_fused": (_I, [_VP, _I64, _I64, _I64, _I64, _I64]),
+    "w4a8_linear_bias": (_I, [_VP, _I64, _VP, _VP, _I, _VP, _VP, _I64, _VP, _I64, _VP, _I64, _I64, _I64, _I64, _VP,
+                              _I64, _VP]),
     "w4a8_linear": (_I, [_VP, _I64, _VP, _VP, _I, _VP, _I64, _VP, _I64, _VP, _I64, _I64, _I64, _I64, _VP, _I64, _VP]),
     "w4a8_midgroup_quant_a": (_I, [_VP, _I64, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _VP]),
     "w4a8_midgroup_gemm": (_I, [_VP, _VP, _VP, _VP, _I64, _I64, _VP, _VP, _VP, _VP, _I64, _VP, _I64, _I64, _I64,

@@ -123,7 +123,7 @@ int check_gemm(const void* a_q, int64_t lda, const void* a_scale, const void* w_
 int run_gemm(const void* a_q, int64_t lda, const void* a_scale, const void* w_tiles,
              const void* s_tiles, int scale_dtype, void* y, int64_t ldy, void* partials,
              int64_t M, int64_t N, int64_t K, int64_t group, void* workspace,
-             int64_t workspace_bytes, void* stream, bool swiglu = false) {
+             int64_t workspace_bytes, void* stream, bool swiglu = false, const void* bias = nullptr) {
     if (int rc = check_gemm(a_q, lda, a_scale, w_tiles, s_tiles, scale_dtype, y, ldy, M, N, K,
                             group, workspace, workspace_bytes, swiglu))
         return rc;
@@ -139,6 +139,7 @@ int run_gemm(const void* a_q, int64_t lda, const void* a_scale, const void* w_ti
     a.ldy = ldy;
     a.partials = static_cast<int32_t*>(partials);
     a.swiglu = swiglu;
+    a.bias = static_cast<const uint16_t*>(bias);
     a.M = M;
     a.N = N;
     a.K = K;
@@ -317,16 +318,16 @@ int w4a8_gemm_swiglu(const void* a_q, int64_t lda, const void* a_scale, const vo
                     workspace, workspace_bytes, stream, true);
 }
 
-int w4a8_linear(const void* x, int64_t ldx, const void* w_tiles, const void* s_tiles, int scale_dtype,
-                void* y, int64_t ldy, void* a_q, int64_t lda, void* a_scale, int64_t M, int64_t N,
-                int64_t K, int64_t group, void* workspace, int64_t workspace_bytes, void* stream) {
+int w4a8_linear_bias(const void* x, int64_t ldx, const void* w_tiles, const void* s_tiles, int scale_dtype,
+                     const void* bias, void* y, int64_t ldy, void* a_q, int64_t lda, void* a_scale, int64_t M,
+                     int64_t N, int64_t K, int64_t group, void* workspace, int64_t workspace_bytes, void* stream) {
     if (int rc = check_gemm(a_q, lda, a_scale, w_tiles, s_tiles, scale_dtype, y, ldy, M, N, K, group, workspace,
                             workspace_bytes, false))
         return rc;
     if (M == 0) return W4A8_OK;
     if (!x) return fail(W4A8_ERR_NULL, "x is NULL");
     if (ldx < K) return fail(W4A8_ERR_SHAPE, "ldx=%lld must be >= K=%lld", ldx, K);
-    if (!aligned(x, 2)) return fail(W4A8_ERR_ALIGN, "x must be 2-byte aligned");
+    if (!aligned(x, 2) || !aligned(bias, 2)) return fail(W4A8_ERR_ALIGN, "x and bias must be 2-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     GemmArgs a{};
     a.a_q = static_cast<const int8_t*>(a_q);
@@ -337,6 +338,7 @@ int w4a8_linear(const void* x, int64_t ldx, const void* w_tiles, const void* s_t
     a.scale_bf16 = scale_dtype == W4A8_DT_BF16;
     a.y = static_cast<uint16_t*>(y);
     a.ldy = ldy;
+    a.bias = static_cast<const uint16_t*>(bias);
     a.M = M;
     a.N = N;
     a.K = K;
@@ -350,7 +352,14 @@ int w4a8_linear(const void* x, int64_t ldx, const void* w_tiles, const void* s_t
                             "w4a8_linear quant launch"))
         return rc;
     return run_gemm(a_q, lda, a_scale, w_tiles, s_tiles, scale_dtype, y, ldy, nullptr, M, N, K, group, workspace,
-                    workspace_bytes, stream);
+                    workspace_bytes, stream, false, bias);
+}
+
+int w4a8_linear(const void* x, int64_t ldx, const void* w_tiles, const void* s_tiles, int scale_dtype,
+                void* y, int64_t ldy, void* a_q, int64_t lda, void* a_scale, int64_t M, int64_t N,
+                int64_t K, int64_t group, void* workspace, int64_t workspace_bytes, void* stream) {
+    return w4a8_linear_bias(x, ldx, w_tiles, s_tiles, scale_dtype, nullptr, y, ldy, a_q, lda, a_scale, M, N, K,
+                            group, workspace, workspace_bytes, stream);
 }
 
 int w4a8_linear_fused(const void* x, int64_t ldx, int64_t M, int64_t N, int64_t K, int64_t group) {

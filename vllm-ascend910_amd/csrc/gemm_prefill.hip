@@ -75,6 +75,7 @@ struct PrefillParams {
     const int8_t* A;
     int64_t lda;
     const uint16_t* a_scale;
+    const uint16_t* bias;   // optional bf16 [N], added to the bf16 outputs on their way out (store_tile)
     const uint4* W;
     const uint16_t* S;
     uint16_t* Y;
@@ -129,18 +130,30 @@ __device__ __forceinline__ void tile_of(const PrefillParams& p, int& tile_m, int
 // elements; rows 0..BM/2-1 from lo, the rest from hi), leaves as 16-byte row
 // stores of 8 columns per thread and step; rows past M are skipped, and a
 // chunk past the last column (or a row that cannot take 16-byte stores) is
-// stored element by element.
+// stored element by element.  bsl holds the bias of the tile's OC columns (read only
+// with p.bias).
 template <int BM, int THREADS, int OC, int OS>
 __device__ __forceinline__ void store_tile(const PrefillParams& p, const uint16_t* lo, const uint16_t* hi, int m0,
-                                           int n0, int ncols, int tid) {
+                                           int n0, int ncols, int tid, const uint16_t* bsl) {
     constexpr int CPR = OC / 8;   // chunks per row
+    static_assert(THREADS % CPR == 0, "a thread's chunks share their columns");
+    uint4 bv = make_uint4(0u, 0u, 0u, 0u);
+    if (p.bias) bv = *reinterpret_cast<const uint4*>(bsl + (tid % CPR) * 8);
+    const uint32_t b[4] = {bv.x, bv.y, bv.z, bv.w};
 #pragma unroll
     for (int k = 0; k < BM * CPR / THREADS; ++k) {
         const int c = tid + k * THREADS;
         const int r = c / CPR, c8 = (c % CPR) * 8;
         const int row = m0 + r, col = n0 + c8;
         if (row >= p.M || col >= ncols) continue;
-        const uint4 v = *reinterpret_cast<const uint4*>((r < BM / 2 ? lo : hi) + (r % (BM / 2)) * OS + c8);
+        uint4 v = *reinterpret_cast<const uint4*>((r < BM / 2 ? lo : hi) + (r % (BM / 2)) * OS + c8);
+        if (p.bias) {
+            uint32_t* pv = reinterpret_cast<uint32_t*>(&v);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                pv[q] = f32x2_to_bf16x2_bits(__uint_as_float(pv[q] << 16) + __uint_as_float(b[q] << 16),
+                                             __uint_as_float(pv[q] & 0xffff0000u) + __uint_as_float(b[q] & 0xffff0000u));
+        }
         uint16_t* y = p.Y + static_cast<int64_t>(row) * p.ldy + col;
         if (p.vec_out && col + 8 <= ncols) {
             *reinterpret_cast<uint4*>(y) = v;
@@ -254,6 +267,13 @@ __global__ __launch_bounds__(threads_for<BM>(), 2) void gemm_prefill_kernel(cons
     uint32_t ts_bits = 0;
     if constexpr (!COMPAT) {
         if (tid < kBM && m0 + tid < p.M) ts_bits = p.a_scale[m0 + tid];
+    }
+    // likewise the bias of the tile's columns (128 columns, at least 128 threads)
+    constexpr bool BIAS = !COMPAT && !SWIGLU && !DUMP;
+    __shared__ __attribute__((aligned(16))) uint16_t bsl[BIAS ? kBN : 8];
+    uint16_t b_bits = 0;
+    if constexpr (BIAS) {
+        if (p.bias && tid < kBN && n0 + tid < p.N) b_bits = p.bias[n0 + tid];
     }
 
     // ---- weights: byte offsets of this lane's two 16-byte chunks per step,
@@ -476,6 +496,9 @@ __global__ __launch_bounds__(threads_for<BM>(), 2) void gemm_prefill_kernel(cons
     // whose fold of row block 1 adds zero partials times zero)
     uint32_t scp[2] = {0u, 0u};
     if (tid < kBM) tsl[tid] = ts_bits;
+    if constexpr (BIAS) {
+        if (tid < kBN) bsl[tid] = b_bits;
+    }
     if constexpr (COMPAT) store_rv(0, rv0);
     // A(0) has landed once at most the loads issued after it are outstanding
     // (A(1), A(2), the weight ring, the scales, the row ring); then every
@@ -707,7 +730,7 @@ __global__ __launch_bounds__(threads_for<BM>(), 2) void gemm_prefill_kernel(cons
     }
     __syncthreads();
     store_tile<kBM, kThreads, OC, OS>(p, reinterpret_cast<const uint16_t*>(la0), reinterpret_cast<const uint16_t*>(la1),
-                                      m0, n0, SWIGLU ? p.half_n : p.N, tid);
+                                      m0, n0, SWIGLU ? p.half_n : p.N, tid, bsl);
 }
 
 constexpr int kDW = 2;   // weight prefetch depth in K steps
@@ -766,6 +789,12 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kerne
     __shared__ __attribute__((aligned(16))) float tsl[kBM];
     uint32_t ts_bits = 0;
     if (tid < kBM && m0 + tid < p.M) ts_bits = p.a_scale[m0 + tid];
+    // the bias of the tile's columns
+    __shared__ __attribute__((aligned(16))) uint16_t bsl[SWIGLU ? 8 : kBN];
+    uint16_t b_bits = 0;
+    if constexpr (!SWIGLU) {
+        if (p.bias && tid < kBN && n0 + tid < p.N) b_bits = p.bias[n0 + tid];
+    }
 
     // weights: this lane's two 16-byte chunks per step of the wave's block
     const int col = SWIGLU ? n0 + (wave & 1) * 32 + c32 + (wave >> 1) * p.half_n : n0 + wave * 32 + c32;
@@ -829,6 +858,9 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kerne
     asm volatile("" ::: "memory");
     uint32_t scp = 0u;   // the previous step's scale (the last row block folds one step late)
     if (tid < kBM) tsl[tid] = bf16_bits_to_f32(ts_bits) * 0.0625f;
+    if constexpr (!SWIGLU) {
+        if (tid < kBN) bsl[tid] = b_bits;
+    }
     wait_vm_barrier<2 * NA + kDW * 2 + 1>();
 
     uint32_t aread[4];
@@ -931,7 +963,7 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_prefill_cols_kerne
     const auto* lo = reinterpret_cast<const uint16_t*>(la0);
     const auto* hi = reinterpret_cast<const uint16_t*>(la1);
     if constexpr (SWIGLU) store_tile_swiglu<kBM, kThreads, OS>(p, lo, hi, m0, n0, tid);
-    else store_tile<kBM, kThreads, OC, OS>(p, lo, hi, m0, n0, p.N, tid);
+    else store_tile<kBM, kThreads, OC, OS>(p, lo, hi, m0, n0, p.N, tid, bsl);
 }
 
 // The reference's mid-group activation planes rebuilt for the compat variant
@@ -1193,6 +1225,7 @@ hipError_t launch_gemm_prefill_split(const GemmArgs& a, int splits, hipStream_t 
     p.A = a.a_q;
     p.lda = a.lda;
     p.a_scale = a.a_scale;
+    p.bias = a.bias;
     p.W = reinterpret_cast<const uint4*>(a.w_tiles);
     p.S = a.s_tiles;
     p.Y = a.y;
@@ -1223,7 +1256,7 @@ hipError_t launch_gemm_prefill_split(const GemmArgs& a, int splits, hipStream_t 
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.splits == 1) return e;
     return launch_split_reduce(p.R, p.ldr, p.a_scale, p.Y, p.ldy, p.M, p.N, p.splits, false, a.scale_bf16, p.S,
-                               nullptr, stream);
+                               nullptr, p.bias, stream);
 }
 
 hipError_t launch_gemm_prefill_bm(const GemmArgs& a, int bm, hipStream_t stream) {
@@ -1232,6 +1265,7 @@ hipError_t launch_gemm_prefill_bm(const GemmArgs& a, int bm, hipStream_t stream)
     p.A = a.a_q;
     p.lda = a.lda;
     p.a_scale = a.a_scale;
+    p.bias = a.bias;
     p.W = reinterpret_cast<const uint4*>(a.w_tiles);
     p.S = a.s_tiles;
     p.Y = a.y;

@@ -35,7 +35,7 @@ using at::Tensor;
 // The C ABI entry points used here, in the order bind() receives their addresses.
 #define W4A8_TORCH_FNS(F)                                                                                     \
     F(w4a8_last_error) F(w4a8_quant_act) F(w4a8_gemm_workspace_bytes) F(w4a8_gemm) F(w4a8_gemm_swiglu)        \
-    F(w4a8_linear) F(w4a8_rmsnorm_quant) F(w4a8_rope_kv) F(w4a8_attention) F(w4a8_attention_rope)             \
+    F(w4a8_linear_bias) F(w4a8_rmsnorm_quant) F(w4a8_rope_kv) F(w4a8_attention) F(w4a8_attention_rope)        \
     F(w4a8_attention_workspace_bytes) F(w4a8_midgroup_quant_a) F(w4a8_midgroup_gemm_workspace_bytes)          \
     F(w4a8_midgroup_tiles_bytes) F(w4a8_midgroup_gemm_ws) F(w4a8_midgroup_gemm_tiled)
 
@@ -181,11 +181,19 @@ Tensor gemm_swiglu(const Tensor& a_q, const Tensor& a_scale, const Tensor& w_til
 }
 
 // ------------------------------------------------------------------ quant + GEMM
-Tensor linear(const Tensor& x0, const Tensor& w_tiles, const Tensor& s_tiles, int64_t N, int64_t K, int64_t group) {
+Tensor linear(const Tensor& x0, const Tensor& w_tiles, const Tensor& s_tiles, int64_t N, int64_t K, int64_t group,
+              const std::optional<Tensor>& bias0) {
     TORCH_CHECK(x0.dim() == 2 && x0.scalar_type() == at::kBFloat16, "w4a8_linear: x must be bfloat16 [M, K]");
     TORCH_CHECK(x0.size(1) == K, "w4a8_linear: x has ", x0.size(1), " columns, K=", K);
     check_geometry("w4a8_linear", K, group);
     check_weights(w_tiles, s_tiles, N, K, group);
+    std::optional<Tensor> bias;
+    if (bias0.has_value()) {
+        TORCH_CHECK(bias0->scalar_type() == at::kBFloat16 && bias0->dim() == 1 && bias0->size(0) == N &&
+                        bias0->device() == x0.device(),
+                    "w4a8_linear: bias must be bfloat16 [N] on the device of x");
+        bias = bias0->contiguous();
+    }
     const Tensor x = rows(x0);
     const int64_t M = x.size(0), width = geom::kpad(K, group);
     Tensor y = empty({M, N}, at::kBFloat16, x);
@@ -197,8 +205,9 @@ Tensor linear(const Tensor& x0, const Tensor& w_tiles, const Tensor& s_tiles, in
     const Abi& f = abi();
     const int64_t need = f.w4a8_gemm_workspace_bytes(M, N, K, group);
     const Workspace ws = need > 0 ? workspace(x, need) : Workspace{};
-    check(f.w4a8_linear(x.data_ptr(), x.stride(0), w_tiles.data_ptr(), s_tiles.data_ptr(), scale_code(s_tiles),
-                        y.data_ptr(), N, p, width, p + as_off, M, N, K, group, ws.ptr, ws.bytes, stream_of(x)),
+    check(f.w4a8_linear_bias(x.data_ptr(), x.stride(0), w_tiles.data_ptr(), s_tiles.data_ptr(), scale_code(s_tiles),
+                             opt_ptr(bias), y.data_ptr(), N, p, width, p + as_off, M, N, K, group, ws.ptr, ws.bytes,
+                             stream_of(x)),
           "w4a8_linear");
     return y;
 }

@@ -29,6 +29,15 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
     return x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
 
 
+def _epilogue_bias(bias: torch.Tensor, x: torch.Tensor, N: int) -> bool:
+    """Whether the GEMM's epilogue can add the bias: a bf16 [N] tensor of x's device that
+    nothing differentiates (the op has no derivative; the torch add has).  Every other bias
+    -- another dtype, a shape that broadcasts, a tensor subclass -- is added by torch."""
+    return (type(bias) in (torch.Tensor, nn.Parameter) and bias.dtype is torch.bfloat16 and bias.shape == (N,)
+            and bias.device == x.device and not (bias.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad._current_level < 0)
+
+
 def linear(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor, N: int, group: int,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x @ W.T with per-token int8 activations and per-group int4 weights.
@@ -36,8 +45,9 @@ def linear(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor, N: int
     The reference's ``w4a8_ops.linear`` (npu_ops/python/w4a8_ops.py:243-252).
     """
     K = x.shape[-1]
-    y = torch.ops.npu.w4a8_linear(_rows(x), w_tiles, s_tiles, N, K, group)
-    if bias is not None:
+    fused = bias is not None and _epilogue_bias(bias, x, N)
+    y = torch.ops.npu.w4a8_linear(_rows(x), w_tiles, s_tiles, N, K, group, bias if fused else None)
+    if bias is not None and not fused:
         y = y + bias
     return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
 

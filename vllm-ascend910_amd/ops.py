@@ -10,7 +10,7 @@ group-size-parameterised ops of this build:
     torch.ops.npu.w4a8_gemm(a_q, a_scale, w_tiles, s_tiles, N, K, group) -> y
     torch.ops.npu.w4a8_gemm_partials(a_q, a_scale, w_tiles, s_tiles, N, K, group) -> (y, partials)
     torch.ops.npu.w4a8_gemm_swiglu(a_q, a_scale, w_tiles, s_tiles, N, K, group) -> y [M, N/2]
-    torch.ops.npu.w4a8_linear(x, w_tiles, s_tiles, N, K, group) -> y   (quant + GEMM)
+    torch.ops.npu.w4a8_linear(x, w_tiles, s_tiles, N, K, group, bias=None) -> y   (quant + GEMM, + bf16 [N] bias)
 
 and two producer-side helpers of the decoder forward that drives them:
 
@@ -65,7 +65,8 @@ _LIB.define("w4a8_gemm_partials(Tensor a_q, Tensor a_scale, Tensor w_tiles, Tens
             "int N, int K, int group) -> (Tensor, Tensor)")
 _LIB.define("w4a8_gemm_swiglu(Tensor a_q, Tensor a_scale, Tensor w_tiles, Tensor s_tiles, "
             "int N, int K, int group) -> Tensor")
-_LIB.define("w4a8_linear(Tensor x, Tensor w_tiles, Tensor s_tiles, int N, int K, int group) -> Tensor")
+_LIB.define("w4a8_linear(Tensor x, Tensor w_tiles, Tensor s_tiles, int N, int K, int group, Tensor? bias=None) "
+            "-> Tensor")
 _LIB.define("w4a8_rmsnorm_quant(Tensor x, Tensor weight, float eps, Tensor? residual=None, int group=0, "
             "bool want_normed=False) -> (Tensor, Tensor, Tensor, Tensor)")
 _LIB.define("w4a8_rope_kv(Tensor qkv, Tensor cos, Tensor sin, Tensor pos, Tensor(a!) k_cache, Tensor(b!) v_cache, "
@@ -272,7 +273,7 @@ def _gemm_partials_fake(a_q, a_scale, w_tiles, s_tiles, N, K, group):
 
 # ---------------------------------------------------------------- quant + GEMM
 @torch.library.register_fake("npu::w4a8_linear")
-def _linear_fake(x, w_tiles, s_tiles, N, K, group):
+def _linear_fake(x, w_tiles, s_tiles, N, K, group, bias=None):
     return x.new_empty((x.shape[0], N), dtype=torch.bfloat16)
 
 

@@ -411,6 +411,22 @@ int w4a8_midgroup_gemm_ws(const void* a_hi, const void* a_lo, const void* a_scal
                           int64_t workspace_bytes, void* stream);
 
 /*
+ * The same GEMM for few rows, its K split over workgroups.  Where
+ * w4a8_midgroup_split_workspace_bytes(Ma, N, K, group) is non-zero (few rows and a K
+ * long enough that the split pays), the exact int32 group sums of every workgroup's
+ * range of whole groups go to the workspace (4-byte aligned, at least that many bytes;
+ * W4A8_ERR_WORKSPACE otherwise) and a second launch folds them in group order: the
+ * outputs of w4a8_midgroup_gemm bit for bit.  Elsewhere the call runs as
+ * w4a8_midgroup_gemm.  w is w_q, or with w_tiled non-zero w4a8_midgroup_tile_weights'
+ * tiles.
+ */
+int64_t w4a8_midgroup_split_workspace_bytes(int64_t Ma, int64_t N, int64_t K, int64_t group);
+int w4a8_midgroup_gemm_split(const void* a_hi, const void* a_lo, const void* a_scale, const void* a_ksum, int64_t Ma,
+                             int64_t ld_as, const void* w, int w_tiled, const void* w_scale, const void* w_zero,
+                             void* y, int64_t ldy, int64_t N, int64_t K, int64_t group, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+
+/*
  * The compat GEMM on a weight reordered once at load time.  The reference
  * reads w_q [N, kpad/2] as stored on every call (its op takes it so,
  * npu_ops/host/midgroup_w4a8_gemm.cpp:45-140); its vLLM method converts

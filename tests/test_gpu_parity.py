@@ -1469,6 +1469,57 @@ def test_midgroup_random_shapes(pkg, dev, M, N, K, G, asym):
     assert np.abs(y32).max() > 0
 
 
+@pytest.mark.parametrize("M,N,K,G,asym", [
+    (8, 200, 8192, 1024, True),        # fewest rows, N off the 128-column workgroups
+    (16, 130, 8200, 4096, False),      # one row tile, ragged last group
+    (17, 2000, 4096, 512, True),       # two row tiles
+    (32, 56, 6208, 128, True),         # one tile a group, 49 groups
+    (33, 1000, 4160, 1024, True),      # four row tiles, a last K tile half padding
+    (64, 128, 27648, 1024, True),      # most rows, more groups a split than one
+])
+def test_midgroup_split_path(pkg, dev, M, N, K, G, asym):
+    """Few rows with K split over workgroups: the reference's fp32 fold order bit for bit,
+    from stored rows and from tiles, equal to w4a8_midgroup_gemm's, and a short or
+    misaligned workspace refused."""
+    say(f"midgroup split M={M} N={N} K={K} G={G} asym={asym}")
+    lib = pkg._abi.lib()
+    need = lib.w4a8_midgroup_split_workspace_bytes(M, N, K, G)
+    assert need > 0, "case not on the split path"
+    xb, codes, sc, zr, a, args = _midgroup_inputs(pkg, dev, M, N, K, G, asym, seed=5 * M + N + K)
+    y = torch.ops.npu.midgroup_w4a8_gemm(*a, *args, K, G, M)
+    tiles = torch.ops.npu.midgroup_tile_weights(args[0], K, G)
+    yt = torch.ops.npu.midgroup_w4a8_gemm_tiled(*a, tiles, *args[1:], N, K, G, M)
+    q, _ = ow.quant_act_midgroup(xb, G)
+    want = ow.f32_to_bf16_bits(ow.gemm_midgroup_fp32(q, tensor_bf16_bits(a[2])[:, :M], codes, sc, zr, G))
+    assert np.array_equal(tensor_bf16_bits(y), want)
+    assert torch.equal(yt.view(torch.int16), y.view(torch.int16))
+    a_hi, a_lo, a_scale, a_ksum = a
+    w_q, w_scale, w_zero = args[0], args[1], args[3]
+    stream = torch.cuda.current_stream().cuda_stream
+    y1 = torch.empty_like(y)
+    rc = lib.w4a8_midgroup_gemm(a_hi.data_ptr(), a_lo.data_ptr(), a_scale.data_ptr(), a_ksum.data_ptr(), M,
+                                a_scale.stride(0), w_q.data_ptr(), w_scale.data_ptr(), w_zero.data_ptr(),
+                                y1.data_ptr(), N, None, N, K, G, stream)
+    assert rc == 0, lib.w4a8_last_error()
+    assert torch.equal(y1.view(torch.int16), y.view(torch.int16))
+    ws = torch.empty(need + 4, dtype=torch.uint8, device=dev)
+    for ptr, nbytes in ((ws.data_ptr(), need - 1), (None, need), (ws.data_ptr() + 2, need)):
+        assert lib.w4a8_midgroup_gemm_split(a_hi.data_ptr(), a_lo.data_ptr(), a_scale.data_ptr(), a_ksum.data_ptr(),
+                                            M, a_scale.stride(0), w_q.data_ptr(), 0, w_scale.data_ptr(),
+                                            w_zero.data_ptr(), y1.data_ptr(), N, N, K, G, ptr, nbytes, stream) == 6
+
+
+def test_midgroup_split_rule(pkg):
+    """Shapes outside the split's rule keep w4a8_midgroup_gemm's plans."""
+    b = pkg._abi.lib().w4a8_midgroup_split_workspace_bytes
+    for shape in ((7, 5120, 27648, 1024), (65, 5120, 27648, 1024), (16, 5120, 6912, 1024), (16, 16384, 27648, 1024),
+                  (32, 5120, 1280, 1024), (32, 5120, 5120, 256), (64, 5120, 27648, 128), (32, 5120, 5120, 8192),
+                  (0, 5120, 27648, 1024)):
+        assert b(*shape) == 0, shape
+    assert b(16, 5120, 27648, 1024) == 27 * 16 * 5120 * 4
+
+
+
 def test_midgroup_prefill_path_without_zero_points(pkg, dev):
     """The C ABI's symmetric call (w_zero NULL: the variant without the zero-point term)
     equals the call with an all-zero w_zero, through w4a8_midgroup_gemm_ws."""

@@ -46,6 +46,9 @@ SIGNATURES = {
     "w4a8_midgroup_gemm": (_I, [_VP, _VP, _VP, _VP, _I64, _I64, _VP, _VP, _VP, _VP, _I64, _VP, _I64, _I64, _I64,
                                 _VP]),
     "w4a8_midgroup_gemm_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64]),
+    "w4a8_midgroup_split_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64]),
+    "w4a8_midgroup_gemm_split": (_I, [_VP, _VP, _VP, _VP, _I64, _I64, _VP, _I, _VP, _VP, _VP, _I64, _I64, _I64, _I64,
+                                      _VP, _I64, _VP]),
     "w4a8_midgroup_tiles_bytes": (_I64, [_I64, _I64, _I64]),
     "w4a8_midgroup_tile_weights": (_I, [_VP, _VP, _I64, _I64, _I64, _VP]),
     "w4a8_midgroup_gemm_tiled": (_I, [_VP, _VP, _VP, _VP, _I64, _I64, _VP, _VP, _VP, _VP, _I64, _VP, _I64, _I64, _I64,

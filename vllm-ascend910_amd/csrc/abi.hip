@@ -406,7 +406,8 @@ int w4a8_midgroup_quant_a(const void* x, int64_t ldx, void* a_hi, void* a_lo, vo
 static int midgroup_gemm_impl(const void* a_hi, const void* a_lo, const void* a_scale, const void* a_ksum,
                               int64_t Ma, int64_t ld_as, const void* w_q, const void* w_scale, const void* w_zero,
                               void* y, int64_t ldy, void* partials, int64_t N, int64_t K, int64_t group,
-                              void* workspace, int64_t workspace_bytes, void* stream, bool w_tiles = false) {
+                              void* workspace, int64_t workspace_bytes, void* stream, bool w_tiles = false,
+                              bool split = false) {
     if (int rc = check_problem(Ma, N, K, group)) return rc;
     if (geom::group_stride(group) % 128 != 0)
         return fail(W4A8_ERR_UNSUPPORTED, "group=%lld: the mid-group path needs ceil_to(group, 64) %% 128 == 0",
@@ -427,7 +428,7 @@ static int midgroup_gemm_impl(const void* a_hi, const void* a_lo, const void* a_
     // Prefill sizes with a workspace: the LDS-tiled prefill waves (no partial
     // dump there; dumps and calls without a workspace take the mid-group kernel)
     const int64_t need = partials ? 0 : midgroup_prefill_workspace_bytes(Ma, N, K, group);
-    const bool prefill = need > 0 && workspace_bytes > 0;
+    const bool prefill = !split && need > 0 && workspace_bytes > 0;
     if (prefill) {
         if (!workspace || workspace_bytes < need || !aligned(workspace, 256))
             return fail(W4A8_ERR_WORKSPACE, "workspace of %lld bytes (256-byte aligned) needed, got %lld", need,
@@ -455,6 +456,16 @@ static int midgroup_gemm_impl(const void* a_hi, const void* a_lo, const void* a_
     a.K = K;
     a.group = group;
     a.w_tiles = w_tiles;
+    if (split) {
+        const int64_t sums = midgroup_split_workspace_bytes(Ma, N, K, group);
+        if (sums > 0) {
+            if (!workspace || workspace_bytes < sums || !aligned(workspace, 4))
+                return fail(W4A8_ERR_WORKSPACE, "workspace of %lld bytes (4-byte aligned) needed, got %lld", sums,
+                            workspace_bytes);
+            return hip_status(launch_gemm_midgroup_split(a, workspace, static_cast<hipStream_t>(stream)),
+                              "w4a8_midgroup_gemm_split launch");
+        }
+    }
     if (prefill)
         return hip_status(launch_gemm_midgroup_prefill(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream)),
                           "w4a8_midgroup_gemm_ws launch");
@@ -493,6 +504,20 @@ int w4a8_midgroup_gemm_tiled(const void* a_hi, const void* a_lo, const void* a_s
     if (workspace_bytes < 0) return fail(W4A8_ERR_WORKSPACE, "workspace_bytes=%lld < 0", workspace_bytes);
     return midgroup_gemm_impl(a_hi, a_lo, a_scale, a_ksum, Ma, ld_as, w_tiles, w_scale, w_zero, y, ldy, partials, N,
                               K, group, workspace, workspace_bytes, stream, true);
+}
+
+int64_t w4a8_midgroup_split_workspace_bytes(int64_t Ma, int64_t N, int64_t K, int64_t group) {
+    if (Ma < 0 || N <= 0 || K <= 0 || group <= 0) return 0;
+    return midgroup_split_workspace_bytes(Ma, N, K, group);
+}
+
+int w4a8_midgroup_gemm_split(const void* a_hi, const void* a_lo, const void* a_scale, const void* a_ksum, int64_t Ma,
+                             int64_t ld_as, const void* w, int w_tiled, const void* w_scale, const void* w_zero,
+                             void* y, int64_t ldy, int64_t N, int64_t K, int64_t group, void* workspace,
+                             int64_t workspace_bytes, void* stream) {
+    if (workspace_bytes < 0) return fail(W4A8_ERR_WORKSPACE, "workspace_bytes=%lld < 0", workspace_bytes);
+    return midgroup_gemm_impl(a_hi, a_lo, a_scale, a_ksum, Ma, ld_as, w, w_scale, w_zero, y, ldy, nullptr, N, K, group,
+                              workspace, workspace_bytes, stream, w_tiled != 0, true);
 }
 
 int w4a8_midgroup_gemm_ws(const void* a_hi, const void* a_lo, const void* a_scale, const void* a_ksum, int64_t Ma,

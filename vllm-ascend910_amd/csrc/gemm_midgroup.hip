@@ -486,6 +486,195 @@ __global__ __launch_bounds__(64 * kShWaves) void gemm_midgroup_shared_kernel(con
         }
 }
 
+// K split over workgroups (a workspace, and the rule of midgroup_split_workspace_bytes):
+// workgroup (x, y) walks the whole groups of K range y for 128 columns, its four
+// waves' two column blocks each sharing the activation planes through LDS as in
+// gemm_midgroup_shared_kernel, and writes every group's exact int32 sum to
+// I[g][row][ldi]; mid_fold_kernel then folds the groups in the reference's order.
+// Without it the activation planes bound these shapes: every pair of column blocks
+// reads them again (16 rows: as many bytes as its weights), on as few workgroups
+// as N has column pairs.  27648 x 5120 at 16 rows: 32.6 us before, now 18.4 (the weights
+// at 3.8 TB/s) + 5.3 for the fold.
+constexpr int kSpP(int mt) { return mt == 1 ? 4 : 2; }   // activation steps in flight
+
+template <int MT>
+__global__ __launch_bounds__(64 * kShWaves) void gemm_midgroup_split_kernel(const MidParams p, int32_t* __restrict__ I,
+                                                                           int64_t ldi) {
+    constexpr int R = 16 * MT, CPW = kShCPW, D = kShD, P = kSpP(MT);
+    static_assert(D == 4 && (P == 2 || P == 4), "the unrolled step indexes the rings statically");
+    // two steps of two tiles, each tile [row block][plane][row][64 B]; thread tid stages
+    // the 16 bytes at tid * 16 of every row block's 4 KB
+    __shared__ __attribute__((aligned(16))) uint8_t ring[2][MT][4096];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = (blockIdx.x * kShWaves + wave) * CPW;
+    const int q = lane >> 4;
+    const int colq = lane & 15;
+    // whole groups [g0, g1) and their tiles (the host keeps splits <= groups)
+    const int g0 = (static_cast<int>(blockIdx.y) * p.NG) / static_cast<int>(gridDim.y);
+    const int g1 = (static_cast<int>(blockIdx.y + 1) * p.NG) / static_cast<int>(gridDim.y);
+    const int ta = g0 * p.tpg, tb = min(p.KT, g1 * p.tpg);
+
+    uint32_t wo[CPW];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) wo[c] = mid_woff(p, (nb + c) * 16 + colq, q);
+    uint4 wb[D][CPW];
+    auto load_w = [&](int s, int t) {
+        const bool half = q >= 2 && (p.kpad - t * 128) < 128;
+        const auto rw = make_rsrc_at(p.w_q, static_cast<uint32_t>(min(t, p.KT - 1)) * mid_wstep(p), t < tb ? p.w_bytes : 0u);
+#pragma unroll
+        for (int c = 0; c < CPW; ++c) wb[s][c] = buf_load16(rw, half ? kOOBm : wo[c]);
+    };
+    const int sts = tid >> 7;
+    const int srow = (tid >> 2) & 15;
+    const uint8_t* splane = ((tid >> 6) & 1) ? p.a_lo : p.a_hi;
+    uint32_t soff[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int row = mt * 16 + srow;
+        soff[mt] = row < p.Ma ? static_cast<uint32_t>(row) * static_cast<uint32_t>(p.kb) + 16u * (tid & 3) : kOOBm;
+    }
+    uint4 ga[P][MT];
+    auto load_a = [&](int slot, int step) {
+        const int t = ta + 2 * step + sts;
+        const auto r = make_rsrc_at(splane, static_cast<uint32_t>(min(t, p.KT - 1)) * 64u, t < tb ? p.a_bytes : 0u);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) ga[slot][mt] = buf_load16(r, soff[mt]);
+    };
+    auto put_a = [&](int slot, int half) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<uint4*>(&ring[half][mt][tid * 16]) = ga[slot][mt];
+    };
+
+    v4i Pm[MT][CPW];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int c = 0; c < CPW; ++c) Pm[mt][c] = v4i{0, 0, 0, 0};
+    auto store = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int c = 0; c < CPW; ++c) {
+                const int col = (nb + c) * 16 + colq;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = mt * 16 + 4 * q + i;
+                    if (r < p.Ma && col < ldi) I[(static_cast<int64_t>(g) * p.Ma + r) * ldi + col] = Pm[mt][c][i] >> 4;
+                }
+                Pm[mt][c] = v4i{0, 0, 0, 0};
+            }
+    };
+
+    const int nsteps = (tb - ta + 1) / 2;
+#pragma unroll
+    for (int i = 0; i < P; ++i) load_a(i, i);
+#pragma unroll
+    for (int s = 0; s < D; ++s) load_w(s, ta + s);
+    put_a(0, 0);
+    load_a(0, P);
+    __syncthreads();   // step 0
+
+    for (int s0 = 0; s0 < nsteps; s0 += P) {
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const int s = s0 + i;
+            if (s >= nsteps) break;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int t = ta + 2 * s + u;
+                if (t >= tb) break;
+                const int ws_slot = (2 * i + u) % D;
+                v4i bw[CPW][2];
+#pragma unroll
+                for (int c = 0; c < CPW; ++c) {
+                    const uint4 w = wb[ws_slot][c];
+                    bw[c][0] = v4i{unpack_lo4(w.x), unpack_hi4(w.x), unpack_lo4(w.y), unpack_hi4(w.y)};
+                    bw[c][1] = v4i{unpack_lo4(w.z), unpack_hi4(w.z), unpack_lo4(w.w), unpack_hi4(w.w)};
+                }
+                load_w(ws_slot, t + D);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const uint8_t* slot = ring[i & 1][mt] + u * 2048 + colq * 64 + q * 16;
+                    const uint4 h = *reinterpret_cast<const uint4*>(slot);
+                    const uint4 l = *reinterpret_cast<const uint4*>(slot + 1024);
+                    int e[4], o[4];
+                    act_pair(h.x, l.x, e[0], o[0]);
+                    act_pair(h.y, l.y, e[1], o[1]);
+                    act_pair(h.z, l.z, e[2], o[2]);
+                    act_pair(h.w, l.w, e[3], o[3]);
+                    const v4i av0 = v4i{e[0], o[0], e[1], o[1]};
+                    const v4i av1 = v4i{e[2], o[2], e[3], o[3]};
+#pragma unroll
+                    for (int c = 0; c < CPW; ++c) Pm[mt][c] = mfma16(av0, bw[c][0], Pm[mt][c]);
+#pragma unroll
+                    for (int c = 0; c < CPW; ++c) Pm[mt][c] = mfma16(av1, bw[c][1], Pm[mt][c]);
+                }
+                if ((t + 1) % p.tpg == 0 || t == tb - 1) store(t / p.tpg);
+            }
+            // step s + 1 into the other half (read last in step s - 1, which every
+            // wave finished before the previous barrier)
+            put_a((i + 1) % P, (i + 1) & 1);
+            load_a((i + 1) % P, s + 1 + P);
+            __syncthreads();
+        }
+    }
+}
+
+// The fold of the split kernel's sums, one output per thread: the zero point's
+// rank-1 term, then (float(I) * ws) * as group by group, the roundings and order
+// of the other kernels.  Latency-bound: the loads of U groups are issued before
+// the first is used (the empty asm keeps the compiler from moving them down to
+// their uses), the row's scales and ksums go through LDS.
+template <bool ASYM, int U>
+__global__ __launch_bounds__(128) void mid_fold_kernel(const MidParams p, const int32_t* __restrict__ I, int64_t ldi) {
+#pragma clang fp contract(off)
+    extern __shared__ float smem[];   // [NG] activation scales, [NG] ksums
+    float* const s_as = smem;
+    int* const s_ak = reinterpret_cast<int*>(smem + p.NG);
+    const int c = static_cast<int>(blockIdx.x) * 128 + static_cast<int>(threadIdx.x);
+    const int col = min(c, p.N - 1);
+    const int row = static_cast<int>(blockIdx.y);
+    int v[U];
+    uint32_t ws[U], wz[U];
+    auto load = [&](int g0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t g = min(g0 + u, p.NG - 1);
+            v[u] = I[(g * p.Ma + row) * ldi + col];
+            ws[u] = p.w_scale[g * p.N + col];
+            wz[u] = ASYM ? p.w_zero[g * p.N + col] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            asm volatile("" : "+v"(v[u]), "+v"(ws[u]));
+            if constexpr (ASYM) asm volatile("" : "+v"(wz[u]));
+        }
+    };
+    for (int g = static_cast<int>(threadIdx.x); g < p.NG; g += 128) {
+        s_as[g] = bf16_bits_to_f32(p.a_scale[static_cast<int64_t>(g) * p.ld_as + row]);
+        s_ak[g] = p.a_ksum[static_cast<int64_t>(g) * p.ld_as + row];
+    }
+    load(0);
+    __syncthreads();
+    float a = 0.0f;
+    for (int g0 = 0;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (g0 + u >= p.NG) break;
+            const int Ig = v[u] + (ASYM ? static_cast<int>(bf16_bits_to_f32(wz[u])) * s_ak[g0 + u] : 0);
+            const float t1 = static_cast<float>(Ig) * bf16_bits_to_f32(ws[u]);
+            a = a + t1 * s_as[g0 + u];
+        }
+        g0 += U;
+        if (g0 >= p.NG) break;
+        load(g0);
+    }
+    if (c < p.N) p.Y[static_cast<int64_t>(row) * p.ldy + c] = static_cast<uint16_t>(f32_to_bf16_bits(a));
+}
+
 // Variants (rows x columns per workgroup, load depth, most waves):
 //   Ma <= 16       16 x 32, depth 4, up to 12 waves (decode)
 //   Ma <= 64       64 x 32, depth 2, up to 8 waves
@@ -649,7 +838,32 @@ int64_t midgroup_lds_bytes(int64_t Ma, int64_t K, int64_t group) {
 
 int64_t midgroup_lds_max() { return static_cast<int64_t>(kMidLdsIsum); }
 
-hipError_t launch_gemm_midgroup(const MidgroupArgs& a, hipStream_t stream) {
+// The shapes whose K is split over workgroups (gemm_midgroup_split_kernel), in us
+// without / with the split (weights from memory, group 1024 unless said):
+//   17-64 rows: the other plan walks K once per 64 x 32 tile, or per 32 x 32 tile
+//     where the group sums of 64 rows exceed the LDS.  K 27648 x N 5120 at 17 / 32 /
+//     64 rows 36.4 / 48.5 / 80.9 against 26.4 / 29.6 / 43.3; 14336 x 4096 22.3 / 27.3 /
+//     39.6 against 13.8 / 14.7 / 20.4; 5120 x 5120 11.5 / 13.6 / 18.8 against 10.1 /
+//     10.6 / 14.1; 5120 x 7168 11.7 / 13.8 / 19.3 against 11.8 / 12.7 / 17.8.  A short K
+//     has too little to split: 1280 x 5120 at 32 rows 8.2 against 9.1.  Below group
+//     stride 512 the sums weigh more: 5120 x 5120 in groups of 256 at 32 rows 14.8
+//     against 15.2, 6912 x 5120 18.2 against 17.1.
+//   8-16 rows: only a long K.  27648 x 5120 at 8 / 16 rows 25.9 / 32.6 against 24.6 /
+//     25.1, 14336 x 4096 12.8 / 15.7 against 12.0 / 12.6; 6912 x 5120 at 8 rows 9.3
+//     against 9.5, 5120 x 7168 at 16 rows 9.7 against 10.6.
+//   Below 8 rows the rows' planes cost little: 27648 x 5120 at 4 rows 22.8 against 23.5.
+// The sums are kept to 128 MiB; wide N has its own plans (the shared-activation
+// kernel, the prefill tiles).
+int64_t midgroup_split_workspace_bytes(int64_t Ma, int64_t N, int64_t K, int64_t group) {
+    if (Ma < 8 || Ma > 64 || (geom::col_blocks(N) + 1) / 2 >= 512) return 0;
+    const int64_t min_k = Ma <= 16 ? 8192 : geom::group_stride(group) >= 512 ? 4096 : 6144;
+    if (K < min_k || geom::num_groups(K, group) < 2) return 0;
+    if (midgroup_prefill_workspace_bytes(Ma, N, K, group) > 0) return 0;
+    const int64_t bytes = geom::num_groups(K, group) * Ma * geom::col_blocks(N) * 16 * 4;
+    return bytes <= (int64_t{128} << 20) ? bytes : 0;
+}
+
+static MidParams mid_params(const MidgroupArgs& a) {
     MidParams p{};
     p.a_hi = static_cast<const uint8_t*>(a.a_hi);
     p.a_lo = static_cast<const uint8_t*>(a.a_lo);
@@ -675,6 +889,41 @@ hipError_t launch_gemm_midgroup(const MidgroupArgs& a, hipStream_t stream) {
     p.wtiles = a.w_tiles;
     p.w_bytes = static_cast<uint32_t>(a.w_tiles ? midgroup_tiles_bytes(a.N, a.K, a.group)
                                                 : a.N * static_cast<int64_t>(p.kb));
+    return p;
+}
+
+hipError_t launch_gemm_midgroup_split(const MidgroupArgs& a, void* workspace, hipStream_t stream) {
+    const MidParams p = mid_params(a);
+    int32_t* I = static_cast<int32_t*>(workspace);
+    const int64_t ldi = static_cast<int64_t>(p.NB) * 16;
+    constexpr int kColBlocks = kShWaves * kShCPW;
+    const unsigned cols = static_cast<unsigned>((p.NB + kColBlocks - 1) / kColBlocks);
+    // two 64-row workgroups a CU (what its registers hold), three of the smaller ones
+    // (27648 x 5120 at 16 / 32 / 64 rows, us: two 25.7 / 30.3 / 43.7, three 25.1 / 29.7 /
+    // 47.7, four 29.6 / 37.1 / 56.7, the last with a slower fold)
+    const int per_cu = p.Ma > 32 ? 2 : 3;
+    const unsigned splits = static_cast<unsigned>(
+        std::max(1, std::min(p.NG, per_cu * device_cu_count() / static_cast<int>(cols))));
+    const dim3 grid(cols, splits), block(64 * kShWaves);
+    if (p.Ma <= 16) gemm_midgroup_split_kernel<1><<<grid, block, 0, stream>>>(p, I, ldi);
+    else if (p.Ma <= 32) gemm_midgroup_split_kernel<2><<<grid, block, 0, stream>>>(p, I, ldi);
+    else gemm_midgroup_split_kernel<4><<<grid, block, 0, stream>>>(p, I, ldi);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    const dim3 fg(static_cast<unsigned>((p.N + 127) / 128), static_cast<unsigned>(p.Ma));
+    const size_t lds = static_cast<size_t>(p.NG) * 8;
+    auto fold = [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        if (a.w_zero) mid_fold_kernel<true, U><<<fg, dim3(128), lds, stream>>>(p, I, ldi);
+        else mid_fold_kernel<false, U><<<fg, dim3(128), lds, stream>>>(p, I, ldi);
+    };
+    if (p.NG <= 8) fold(std::integral_constant<int, 8>{});
+    else if (p.NG <= 16) fold(std::integral_constant<int, 16>{});
+    else fold(std::integral_constant<int, 32>{});
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_midgroup(const MidgroupArgs& a, hipStream_t stream) {
+    const MidParams p = mid_params(a);
     // waves per workgroup: about two groups each, more for few column blocks
     const int64_t wgs = (p.NB + 1) / 2;
     const int kw = wgs >= 512 ? 1 : std::max(1, std::min(p.NG, static_cast<int>((p.NG + 1) / 2)));

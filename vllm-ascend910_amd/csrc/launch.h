@@ -134,6 +134,11 @@ struct MidgroupArgs {
 int64_t midgroup_lds_bytes(int64_t Ma, int64_t K, int64_t group);
 int64_t midgroup_lds_max();
 hipError_t launch_gemm_midgroup(const MidgroupArgs& a, hipStream_t stream);
+// The same GEMM at up to 64 rows with K split over workgroups: int32 group sums
+// in a workspace of midgroup_split_workspace_bytes (0: the shape takes
+// launch_gemm_midgroup), folded by a second launch.  The same outputs bit for bit.
+int64_t midgroup_split_workspace_bytes(int64_t Ma, int64_t N, int64_t K, int64_t group);
+hipError_t launch_gemm_midgroup_split(const MidgroupArgs& a, void* workspace, hipStream_t stream);
 // The same GEMM at prefill sizes on gemm_prefill_kernel's LDS-tiled waves
 // (gemm_prefill.hip): the activation planes rebuilt into a workspace of
 // midgroup_prefill_workspace_bytes (0: the shape takes launch_gemm_midgroup;

@@ -37,7 +37,8 @@ using at::Tensor;
     F(w4a8_last_error) F(w4a8_quant_act) F(w4a8_gemm_workspace_bytes) F(w4a8_gemm) F(w4a8_gemm_swiglu)        \
     F(w4a8_linear_bias) F(w4a8_rmsnorm_quant) F(w4a8_rope_kv) F(w4a8_attention) F(w4a8_attention_rope)        \
     F(w4a8_attention_workspace_bytes) F(w4a8_midgroup_quant_a) F(w4a8_midgroup_gemm_workspace_bytes)          \
-    F(w4a8_midgroup_tiles_bytes) F(w4a8_midgroup_gemm_ws) F(w4a8_midgroup_gemm_tiled)
+    F(w4a8_midgroup_split_workspace_bytes) F(w4a8_midgroup_gemm_split) F(w4a8_midgroup_tiles_bytes)           \
+    F(w4a8_midgroup_gemm_ws) F(w4a8_midgroup_gemm_tiled)
 
 struct Abi {
 #define W4A8_DECL(n) decltype(&::n) n;
@@ -429,11 +430,21 @@ Tensor run_midgroup(const Tensor& a_hi0, const Tensor& a_lo0, const Tensor& a_sc
     Tensor y = empty({M, N}, at::kBFloat16, a_hi);
     if (M == 0) return y;
     // w_ksum is validated but not read: the activation bytes are rebuilt exactly from
-    // the two planes, so the kernel needs no +8 correction.  Prefill sizes get a
-    // workspace for the rebuilt rows, allocated per call as the reference host
-    // allocates its GEMM workspace (npu_ops/host/midgroup_w4a8_gemm.cpp:116-118).
-    const int64_t need = f.w4a8_midgroup_gemm_workspace_bytes(M, N, K, group);
+    // the two planes, so the kernel needs no +8 correction.  Few rows on a long K get a
+    // workspace for the int32 group sums of a split K, prefill sizes one for the rebuilt
+    // rows, allocated per call as the reference host allocates its GEMM workspace
+    // (npu_ops/host/midgroup_w4a8_gemm.cpp:116-118).
     Tensor ws;
+    if (const int64_t sums = f.w4a8_midgroup_split_workspace_bytes(M, N, K, group)) {
+        ws = empty({sums}, at::kByte, a_hi);
+        check(f.w4a8_midgroup_gemm_split(a_hi.data_ptr(), a_lo.data_ptr(), a_scale.data_ptr(), a_ksum.data_ptr(), M,
+                                         a_scale.stride(0), w_q.data_ptr(), tiled, w_scale.data_ptr(),
+                                         w_zero.data_ptr(), y.data_ptr(), N, N, K, group, ws.data_ptr(), sums,
+                                         stream_of(a_hi)),
+              "midgroup_w4a8_gemm");
+        return y;
+    }
+    const int64_t need = f.w4a8_midgroup_gemm_workspace_bytes(M, N, K, group);
     if (need) ws = empty({need}, at::kByte, a_hi);
     check((tiled ? f.w4a8_midgroup_gemm_tiled : f.w4a8_midgroup_gemm_ws)(
               a_hi.data_ptr(), a_lo.data_ptr(), a_scale.data_ptr(), a_ksum.data_ptr(), M, a_scale.stride(0),

@@ -64,7 +64,7 @@ def test_strided_inputs(pkg, dev, M):
     (130, 1000, 1024, 64),     # 64 x 64 wave tiles
 ])
 def test_linear_bias(pkg, dev, M, N, K, G):
-    """The epilogue's bias on every plan: the bits of the bf16 add after the linear."""
+    """The bias on every plan (past 64 rows in the epilogue): the bits of the bf16 add after the linear."""
     w, s = _weight(dev, N, K, G, M + N)
     x = torch.randn((M, K), device=dev).to(torch.bfloat16)
     bias = torch.randn((N,), device=dev).to(torch.bfloat16)

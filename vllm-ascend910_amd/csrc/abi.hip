@@ -327,6 +327,9 @@ int w4a8_linear_bias(const void* x, int64_t ldx, const void* w_tiles, const void
     if (M == 0) return W4A8_OK;
     if (!x) return fail(W4A8_ERR_NULL, "x is NULL");
     if (ldx < K) return fail(W4A8_ERR_SHAPE, "ldx=%lld must be >= K=%lld", ldx, K);
+    if (bias && M <= kDecodeMaxM)
+        return fail(W4A8_ERR_UNSUPPORTED, "M=%lld: a bias needs more than %lld rows (the prefill kernels add it)", M,
+                    static_cast<long long>(kDecodeMaxM));
     if (!aligned(x, 2) || !aligned(bias, 2)) return fail(W4A8_ERR_ALIGN, "x and bias must be 2-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     GemmArgs a{};
@@ -338,7 +341,6 @@ int w4a8_linear_bias(const void* x, int64_t ldx, const void* w_tiles, const void
     a.scale_bf16 = scale_dtype == W4A8_DT_BF16;
     a.y = static_cast<uint16_t*>(y);
     a.ldy = ldy;
-    a.bias = static_cast<const uint16_t*>(bias);
     a.M = M;
     a.N = N;
     a.K = K;

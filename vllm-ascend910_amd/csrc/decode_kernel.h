@@ -40,7 +40,6 @@ struct DecodeParams {
     const int8_t* A;
     int64_t lda;
     const uint16_t* a_scale;
-    const uint16_t* bias;   // optional bf16 [N], added to the bf16 outputs
     const uint4* W;
     const uint16_t* S;
     uint16_t* Y;
@@ -176,17 +175,6 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
     if constexpr (!QF) {
         if (static_cast<int>(threadIdx.x) < R && m0 + static_cast<int>(threadIdx.x) < p.M)
             ts_bits = p.a_scale[m0 + threadIdx.x];
-    }
-
-    // The bias of the workgroup's columns, likewise requested here.
-    constexpr bool BIAS = !SWIGLU && !DUMP;
-    __shared__ uint32_t bsl[BIAS ? C : 1];
-    uint32_t b_bits = 0;
-    if constexpr (BIAS) {
-        if (p.bias && static_cast<int>(threadIdx.x) < C) {
-            const int col = nb0 * 16 + static_cast<int>(threadIdx.x);
-            if (col < p.N) b_bits = p.bias[col];
-        }
     }
 
     // This wave's tile range [ta, tb).
@@ -627,9 +615,6 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
     if constexpr (!QF) {
         if (static_cast<int>(threadIdx.x) < R) tsc[threadIdx.x] = ts_bits;
     }
-    if constexpr (BIAS) {
-        if (static_cast<int>(threadIdx.x) < C) bsl[threadIdx.x] = b_bits;
-    }
     __syncthreads();
     // the fp32 sum (before the token scale) of local element e = row * C + cc
     auto colsum = [&](int e, int cc) -> float {
@@ -666,11 +651,7 @@ __device__ __forceinline__ void decode_body(const DecodeParams& p) {
             const float sum = colsum(e, e - row * C);
             const uint32_t tsb = QF ? reinterpret_cast<const uint32_t*>(lds + lq_s)[row] : tsc[row];
             const float ts = bf16_bits_to_f32(tsb) * 0.0625f;
-            uint32_t o = f32_to_bf16_bits(sum * ts);
-            if constexpr (BIAS) {
-                if (p.bias) o = add_bias_bits(o, bsl[e - row * C]);
-            }
-            p.Y[static_cast<int64_t>(m0 + row) * p.ldy + col] = static_cast<uint16_t>(o);
+            p.Y[static_cast<int64_t>(m0 + row) * p.ldy + col] = static_cast<uint16_t>(f32_to_bf16_bits(sum * ts));
         }
     }
 }

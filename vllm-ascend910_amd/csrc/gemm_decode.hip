@@ -52,7 +52,6 @@ DecodeParams make_params(const GemmArgs& a) {
     p.A = a.a_q;
     p.lda = a.lda;
     p.a_scale = a.a_scale;
-    p.bias = a.bias;
     p.W = reinterpret_cast<const uint4*>(a.w_tiles);
     p.S = a.s_tiles;
     p.Y = a.y;

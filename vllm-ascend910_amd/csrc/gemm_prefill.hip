@@ -1225,7 +1225,6 @@ hipError_t launch_gemm_prefill_split(const GemmArgs& a, int splits, hipStream_t 
     p.A = a.a_q;
     p.lda = a.lda;
     p.a_scale = a.a_scale;
-    p.bias = a.bias;
     p.W = reinterpret_cast<const uint4*>(a.w_tiles);
     p.S = a.s_tiles;
     p.Y = a.y;
@@ -1256,7 +1255,7 @@ hipError_t launch_gemm_prefill_split(const GemmArgs& a, int splits, hipStream_t 
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.splits == 1) return e;
     return launch_split_reduce(p.R, p.ldr, p.a_scale, p.Y, p.ldy, p.M, p.N, p.splits, false, a.scale_bf16, p.S,
-                               nullptr, p.bias, stream);
+                               nullptr, stream);
 }
 
 hipError_t launch_gemm_prefill_bm(const GemmArgs& a, int bm, hipStream_t stream) {

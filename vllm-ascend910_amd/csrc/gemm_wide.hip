@@ -39,7 +39,6 @@ struct WideParams {
     const int8_t* A;
     int64_t lda;
     const uint16_t* a_scale;
-    const uint16_t* bias;   // optional bf16 [N], added to the bf16 outputs
     const uint4* W;
     const uint16_t* S;
     uint16_t* Y;
@@ -107,16 +106,6 @@ __global__ __launch_bounds__(64 * kWN) void gemm_wide_kernel(const WideParams p)
     __shared__ uint32_t tsc[16 * kMT];
     uint32_t ts_bits = 0;
     if (tid < 16 * kMT && tid < p.M) ts_bits = p.a_scale[tid];
-    // The bias of the workgroup's columns, likewise (one split: the reduce adds it).
-    constexpr bool BIAS = !SWIGLU && !DUMP;
-    constexpr int kCols = 16 * kCPW * kWN;
-    static_assert(kCols <= 64 * kWN, "one bias column per thread");
-    __shared__ uint32_t bsl[BIAS ? kCols : 1];
-    uint32_t b_bits = 0;
-    if constexpr (BIAS) {
-        const int col = static_cast<int>(blockIdx.x) * kCols + tid;
-        if (p.bias && tid < kCols && col < p.N) b_bits = p.bias[col];
-    }
 
     // This workgroup's K range [ta, tb): group-aligned units split evenly
     // (the host keeps splits <= units, so every range is non-empty).
@@ -324,9 +313,6 @@ __global__ __launch_bounds__(64 * kWN) void gemm_wide_kernel(const WideParams p)
         }
     }
     if (tid < 16 * kMT) tsc[tid] = ts_bits;
-    if constexpr (BIAS) {
-        if (tid < kCols) bsl[tid] = b_bits;
-    }
     __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt)
@@ -358,12 +344,9 @@ __global__ __launch_bounds__(64 * kWN) void gemm_wide_kernel(const WideParams p)
 #pragma unroll
                 for (int c = 0; c < kCPW; ++c) {
                     const int col = block_of(c) * 16 + colq;
-                    if (col >= p.N) continue;
-                    uint32_t o = f32_to_bf16_bits(acc[mt][c][q] * ts);
-                    if constexpr (BIAS) {
-                        if (p.bias) o = add_bias_bits(o, bsl[(wn * kCPW + c) * 16 + colq]);
-                    }
-                    p.Y[static_cast<int64_t>(row) * p.ldy + col] = static_cast<uint16_t>(o);
+                    if (col < p.N)
+                        p.Y[static_cast<int64_t>(row) * p.ldy + col] =
+                            static_cast<uint16_t>(f32_to_bf16_bits(acc[mt][c][q] * ts));
                 }
             }
         }
@@ -374,25 +357,18 @@ __global__ __launch_bounds__(64 * kWN) void gemm_wide_kernel(const WideParams p)
 // columns from N to ldr are never written.  ONE (a single group over K): R
 // holds int32 sums, added exactly and then folded with the column scale
 // (s_tiles of one group are indexed by column), and the dump P, if given,
-// receives the group's partial.  bias (optional) is added to the bf16 outputs.
+// receives the group's partial.
 template <bool ONE, bool SBF16>
 __global__ __launch_bounds__(256) void wide_reduce_kernel(const float* __restrict__ R, int64_t ldr,
                                                           const uint16_t* a_scale, uint16_t* Y, int64_t ldy, int M,
-                                                          int N, int splits, const uint16_t* S, int32_t* P,
-                                                          const uint16_t* bias) {
+                                                          int N, int splits, const uint16_t* S, int32_t* P) {
     const int n4 = static_cast<int>(ldr >> 2);
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= static_cast<int64_t>(M) * n4) return;
     const int row = static_cast<int>(idx / n4);
     const int col = static_cast<int>(idx - static_cast<int64_t>(row) * n4) * 4;
     if (col >= N) return;
-    // the token scale and bias are requested with the sums, not after them
-    const uint32_t tsb = a_scale[row];
-    uint32_t bb[4] = {0u, 0u, 0u, 0u};
-    if (bias) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) bb[c] = bias[min(col + c, N - 1)];
-    }
+    const uint32_t tsb = a_scale[row];   // requested with the sums, not after them
     const int64_t plane = static_cast<int64_t>(M) * ldr;
     const float* r = R + static_cast<int64_t>(row) * ldr + col;
     // all loads first (one memory latency, not one per split), then the sum
@@ -435,14 +411,8 @@ __global__ __launch_bounds__(256) void wide_reduce_kernel(const float* __restric
         }
     }
     const float ts = bf16_bits_to_f32(tsb) * 0.0625f;
-    uint32_t o[4] = {f32_to_bf16_bits(s.x * ts), f32_to_bf16_bits(s.y * ts), f32_to_bf16_bits(s.z * ts),
-                     f32_to_bf16_bits(s.w * ts)};
-    if (bias) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) o[c] = add_bias_bits(o[c], bb[c]);
-    }
-    const uint32_t lo = o[0] | (o[1] << 16);
-    const uint32_t hi = o[2] | (o[3] << 16);
+    const uint32_t lo = f32_to_bf16_bits(s.x * ts) | (f32_to_bf16_bits(s.y * ts) << 16);
+    const uint32_t hi = f32_to_bf16_bits(s.z * ts) | (f32_to_bf16_bits(s.w * ts) << 16);
     uint16_t* y = Y + static_cast<int64_t>(row) * ldy + col;
     if (col + 4 <= N && (reinterpret_cast<uintptr_t>(y) & 7u) == 0) {
         *reinterpret_cast<uint2*>(y) = make_uint2(lo, hi);
@@ -496,7 +466,6 @@ WideParams make_wide_params(const GemmArgs& a, int splits) {
     p.A = a.a_q;
     p.lda = a.lda;
     p.a_scale = a.a_scale;
-    p.bias = a.bias;
     p.W = reinterpret_cast<const uint4*>(a.w_tiles);
     p.S = a.s_tiles;
     p.Y = a.y;
@@ -549,24 +518,22 @@ hipError_t launch_wide_v(const GemmArgs& a, WideParams p, hipStream_t stream) {
     else e = launch_gm<kMT, kCPW, kD, kRA, false, false>(p, c, a.scale_bf16, stream);
     if (e != hipSuccess || p.splits == 1) return e;
     return launch_split_reduce(p.R, p.ldr, p.a_scale, p.Y, p.ldy, p.M, p.N, p.splits, p.NG == 1, a.scale_bf16, p.S,
-                               p.P, p.bias, stream);
+                               p.P, stream);
 }
 
 }  // namespace
 
 hipError_t launch_split_reduce(const float* R, int64_t ldr, const uint16_t* a_scale, uint16_t* Y, int64_t ldy, int M,
                                int N, int splits, bool one, bool sbf16, const uint16_t* S, int32_t* P,
-                               const uint16_t* bias, hipStream_t stream) {
+                               hipStream_t stream) {
     const int64_t n = static_cast<int64_t>(M) * (ldr / 4);
     const dim3 rg(static_cast<unsigned>((n + 255) / 256));
     if (one) {
-        if (sbf16)
-            wide_reduce_kernel<true, true><<<rg, 256, 0, stream>>>(R, ldr, a_scale, Y, ldy, M, N, splits, S, P, bias);
-        else
-            wide_reduce_kernel<true, false><<<rg, 256, 0, stream>>>(R, ldr, a_scale, Y, ldy, M, N, splits, S, P, bias);
+        if (sbf16) wide_reduce_kernel<true, true><<<rg, 256, 0, stream>>>(R, ldr, a_scale, Y, ldy, M, N, splits, S, P);
+        else wide_reduce_kernel<true, false><<<rg, 256, 0, stream>>>(R, ldr, a_scale, Y, ldy, M, N, splits, S, P);
     } else {
         wide_reduce_kernel<false, false><<<rg, 256, 0, stream>>>(R, ldr, a_scale, Y, ldy, M, N, splits, nullptr,
-                                                                  nullptr, bias);
+                                                                  nullptr);
     }
     return hipGetLastError();
 }

@@ -141,6 +141,40 @@ def test_large_scores_and_scale(pkg, dev):
             assert torch.equal(pre, attn(q, k, vt, pos0, L, cps, True, scale))
 
 
+@pytest.mark.parametrize("D,q_scale,scale", [(128, 1e9, None), (128, 1e10, -0.2), (64, 1e11, None), (128, 1e12, None),
+                                             (64, 1e12, -0.2), (128, 1e18, 3.0)])
+def test_huge_scores(pkg, dev, D, q_scale, scale):
+    """Finite queries and keys whose scaled scores reach 2^31 and more: the exponent of a row's
+    largest score has to be exactly 0 there (a rounding step of such a score is past the range
+    of 2^x), on both launches and on the fused rotary one.  The rows' two largest scores lie
+    further apart (checked) than the rounding of fp32 sums of D products: the weights are one
+    and zeros, and check()'s bound is one rounding of the best key's value."""
+    B, T, H, KVH = 2, 40, 8, 2
+    say(f"attention huge scores D={D} q x {q_scale:g} scale={scale}")
+    q, k, vt, Lc = make_inputs(dev, B, T, H, KVH, D, 70, seed=17, q_scale=q_scale)
+    s = torch.einsum("bthgd,bhld->bthgl", q.double().cpu().view(B, T, KVH, H // KVH, D), k.double().cpu())
+    s = s * (scale if scale is not None else 1.0 / math.sqrt(D))
+    for t in range(T):
+        if t:
+            top = torch.topk(s[:, t, ..., :t + 1], 2, dim=-1).values
+            assert torch.all(top[..., 0] - top[..., 1] > D * 2.0 ** -24 * s[:, t, ..., :t + 1].abs().amax(-1))
+    ref, mag = reference(q, k, vt, 0, 70, scale)
+    pos0 = torch.zeros((1,), dtype=torch.int64, device=dev)
+    for cps in (1, 2):
+        pre = attn(q, k, vt, pos0, 70, cps, False, scale)
+        check(pre, ref, mag, f"cps={cps}")
+        assert torch.equal(pre, attn(q, k, vt, pos0, 70, cps, True, scale)), f"split launch differs (cps={cps})"
+    # the fused rotary launch at position 0 (angle 0: no rotation) over one earlier key per call
+    qkv = torch.randn((B, (H + 2 * KVH) * D), generator=torch.Generator(device=dev).manual_seed(3), device=dev)
+    qkv[:, :H * D] *= q_scale
+    qkv = qkv.to(torch.bfloat16)
+    one, zero = torch.ones((70, D // 2), device=dev), torch.zeros((70, D // 2), device=dev)
+    p = torch.full((1,), 69, dtype=torch.int64, device=dev)
+    got = torch.ops.npu.w4a8_attention_rope(qkv, one, zero, p, k, vt, H, KVH, 70, 1, None, scale)
+    ref, mag = reference(qkv[:, :H * D].reshape(B, 1, H, D), k, vt, 69, 70, scale)   # k and v now hold the step's
+    check(got, ref, mag, "rotary")
+
+
 @pytest.mark.parametrize("B,T,H,KVH,D,scale,note", [
     (8, 181, 40, 8, 128, None, "two row tiles per wave, a ragged last workgroup"),
     (8, 181, 40, 8, 64, -0.2, "the same at D = 64, a negative scale"),

@@ -14,15 +14,11 @@
 // Arithmetic of a row, in chunks of 64 positions:
 //   scores  S^T = K . Q^T by v_mfma_f32_16x16x32_bf16 (keys as the A rows, the
 //           16 query rows of a tile as the B columns) in fp32, times
-//           c = log2(e) * |scale| (a negative scale flips the queries' signs
-//           instead, exact); positions past p(r) are -inf;
+//           c = log2(e) * scale, rounded to fp32; positions past p(r) are -inf;
 //   chunk   flash update of the running state (m, l, O) of the split the
 //           chunk belongs to: m' = max(m, max_k s), alpha = 2^(m - m'),
-//           P = 2^(s - m') (s - m' as one fused multiply-add of the score),
-//           l' = l * alpha + sum_k P, O' = O * alpha + bf16(P) . V (MFMA: V^T
-//           as the A rows, P^T as the B columns).  l is held per lane (each
-//           of a row's four lanes sums its own 16 positions of a chunk) and
-//           the four meet once, when the split ends;
+//           P = 2^(s - m'), l' = l * alpha + sum_k P, O' = O * alpha +
+//           bf16(P) . V (MFMA: V^T as the A rows, P^T as the B columns);
 //   splits  `cps` consecutive chunks form a split; split states are combined
 //           in the order s = 0, 1, ... by (m1, l1, O1) (+) (m2, l2, O2) =
 //           (m, l1 a1 + l2 a2, O1 a1 + O2 a2), m = max(m1, m2), a_i = 2^(m_i - m);
@@ -81,7 +77,7 @@ struct VOps {
 };
 
 // Running state of one query row.  The row's four lanes (c, j = 0..3) each
-// hold m, their share of l (all of it after state_close) and the slice
+// hold m and l and the slice
 // O^T[16 dt + 4 j + e][c], e = 0..3, of its O.
 template <int D>
 struct RowState {
@@ -129,12 +125,6 @@ __device__ __forceinline__ float row_reduce(float x, F f) {
     const uint32_t v = __float_as_uint(f(__uint_as_float(a[0]), __uint_as_float(a[1])));
     const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
     return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
-// The end of a split: l of the row's four lanes added.
-template <int D>
-__device__ __forceinline__ void state_close(RowState<D>& s) {
-    s.l = row_reduce(s.l, [](float p, float q) { return p + q; });
 }
 
 // s = s (+) t; an empty state (l == 0: no position of the row in that split) is
@@ -189,11 +179,6 @@ __device__ __forceinline__ int last_pos(const AttnArgs& a, int64_t pos0, int r1)
     return clamp_pos(pos0 + min(r1, a.G * a.T - 1) / a.G, a.L);
 }
 
-// Eight bf16 with their signs flipped where flip is 0x80008000 (0: unchanged).
-__device__ __forceinline__ uint4 flip_sign(uint4 v, uint32_t flip) {
-    return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip);
-}
-
 // Q^T as the B operand of the score MFMAs: lane (c, j) holds q[r][32 i + 8 j .. +8]
 // for k-step i; rows past the problem read zero.
 template <int D>
@@ -202,7 +187,7 @@ __device__ __forceinline__ void load_q(const AttnArgs& a, const Tile& t, int j, 
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) {
         const uint4 v = t.real ? *reinterpret_cast<const uint4*>(qr + 32 * i + 8 * j) : make_uint4(0, 0, 0, 0);
-        qop[i] = __builtin_bit_cast(bf16x8, flip_sign(v, a.qflip));
+        qop[i] = __builtin_bit_cast(bf16x8, v);
     }
 }
 
@@ -244,7 +229,12 @@ __device__ __forceinline__ void chunk_scores(f32x4 (&sc)[4], const bf16x8 (&qop)
 
 // The softmax update of one chunk (positions c0 ..): m and l of the state, the
 // factor alpha of its O, and P^T as the B operands of the chunk's two key
-// blocks.  MASK: the chunk may hold positions past p_row.  cs > 0.
+// blocks.  MASK: the chunk may hold positions past p_row.
+//
+// The exponent of a score is the difference of two rounded products, so that of
+// the row's largest is exactly 0 at any size of the scores; one fused
+// multiply-add of the raw score would leave the rounding error of m there, which
+// from |m| = 2^31 on drives every probability of a row to 0 or infinity.
 template <bool MASK>
 __device__ __forceinline__ void chunk_softmax(float& m, float& l, float& alpha, bf16x8 (&pop)[2],
                                               const f32x4 (&sc)[4], int c0, int p_row, float cs, int j) {
@@ -254,25 +244,27 @@ __device__ __forceinline__ void chunk_softmax(float& m, float& l, float& alpha, 
     for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            x[kt][e] = (!MASK || lane_pos(kt, 0, e) <= p_row - c0 - 8 * j) ? sc[kt][e] : -INFINITY;
+            x[kt][e] = (!MASK || lane_pos(kt, 0, e) <= p_row - c0 - 8 * j) ? sc[kt][e] * cs : -INFINITY;
         mt[kt] = vmax(vmax(x[kt][0], x[kt][1]), x[kt][2]);
     }
     mt[0] = vmax(vmax(mt[0], x[0][3]), x[1][3]);
     mt[2] = vmax(vmax(mt[2], x[2][3]), x[3][3]);
     mt[0] = vmax(vmax(mt[0], mt[1]), vmax(mt[2], mt[3]));
-    const float xm = row_reduce(mt[0], [](float p, float q) { return vmax(p, q); }) * cs;
-    const float mn = vmax(m, xm);
+    const float mn = vmax(m, row_reduce(mt[0], [](float p, float q) { return vmax(p, q); }));
     const float mz = mn == -INFINITY ? 0.0f : mn;   // no position of the row yet: everything stays 0
     // an empty state needs no factor (its l and O are 0)
     alpha = m != -INFINITY ? exp2_neg(m - mz) : 1.0f;
-    float p[4][4], ls[4];
+    float p[4][4];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
+    for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) p[kt][e] = exp2_neg(fmaf(x[kt][e], cs, -mz));
-        ls[kt] = (p[kt][0] + p[kt][1]) + (p[kt][2] + p[kt][3]);
-    }
-    l = fmaf(l, alpha, (ls[0] + ls[1]) + (ls[2] + ls[3]));
+        for (int e = 0; e < 4; ++e) p[kt][e] = exp2_neg(x[kt][e] - mz);
+    float ls = 0.0f;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ls = ls + p[kt][e];
+    l = fmaf(l, alpha, row_reduce(ls, [](float a, float b) { return a + b; }));
     m = mn;
     // P^T as the B operand of key block s: slots 0..7 = positions 32 s + 8 j + 0..7
 #pragma unroll
@@ -478,7 +470,7 @@ __global__ __launch_bounds__(64) void attn_split_kernel(const AttnArgs a) {
         rope_rotate<D>(xk, bk, has_bias, cs, sn, knew);
 #pragma unroll
         for (int i = 0; i < D / 32; ++i)
-            qop[i] = __builtin_bit_cast(bf16x8, (inside && t.real) ? flip_sign(yq[i], a.qflip) : make_uint4(0, 0, 0, 0));
+            qop[i] = __builtin_bit_cast(bf16x8, (inside && t.real) ? yq[i] : make_uint4(0, 0, 0, 0));
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt)
             vnew[dt] = has_bias ? f32_to_bf16_bits(rope_in(xv[dt], bv[dt], true)) : xv[dt];
@@ -539,7 +531,6 @@ __global__ __launch_bounds__(64) void attn_split_kernel(const AttnArgs a) {
         ++ch;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the skipped prefetch
-    state_close(st);
     if (a.ns == 1) {
         write_out<D>(a, t, st, j);
         return;
@@ -626,14 +617,13 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const AttnArgs a) {
 // lanes fall in distinct banks.
 //
 // What bounds it: the vector instructions of the softmax.  Per 16-row tile and
-// chunk there are 32 MFMAs (16 cycles each) and about 80 vector instructions off
+// chunk there are 32 MFMAs (16 cycles each) and about 85 vector instructions off
 // the diagonal (16 exponentials at two issue slots), 32 more where a row's
 // maximum moves; 40 heads of 128 over 8 KV heads, one sequence: 4096 tokens
-// 279 -> 195 us, 8192 tokens 704 us = 0.98 PFLOP/s where a large bf16 matrix
+// 283 -> 192 us, 0.90 PFLOP/s where a large bf16 matrix
 // product reaches 1.19 on the same card.  What it took: two row tiles per wave
 // (one operand read serves two), masks only on the chunks that need them, lane
-// swaps instead of LDS permutes, the maximum on the raw scores and one fused
-// multiply-add per exponent.  Slower at 4096 tokens: the softmax of one tile
+// swaps instead of LDS permutes.  Slower at 4096 tokens: the softmax of one tile
 // placed between the MFMAs of the other in one wave (235 us), eight waves of
 // one tile (202), the folded split states in scratch (233: its loads wait
 // behind the chunk prefetch).
@@ -737,7 +727,6 @@ __global__ __launch_bounds__(64 * kLoopWaves, 2) void attn_loop_kernel(const Att
     for (int t = 0; t < RT; ++t) state_clear(tot[t]);
     auto end_split = [&](int t, int ch) __attribute__((always_inline)) {
         if ((ch + 1) % a.cps == 0 || ch + 1 == nchunks) {
-            state_close(st[t]);
             state_fold<D>(tot[t], st[t]);
             state_clear(st[t]);
         }
@@ -824,13 +813,8 @@ hipError_t launch_attention_d(const AttnArgs& a, bool split, hipStream_t stream)
 
 }  // namespace
 
-hipError_t launch_attention(const AttnArgs& a0, bool split, hipStream_t stream) {
-    if (static_cast<int64_t>(a0.B) * a0.T == 0) return hipSuccess;
-    AttnArgs a = a0;
-    a.qflip = a.cs < 0.0f ? 0x80008000u : 0u;
-    // a factor of 0 (every score 0) as the smallest normal one: the same scores, but
-    // a masked position's -inf stays -inf
-    a.cs = fmaxf(fabsf(a.cs), 1.17549435e-38f);
+hipError_t launch_attention(const AttnArgs& a, bool split, hipStream_t stream) {
+    if (static_cast<int64_t>(a.B) * a.T == 0) return hipSuccess;
     if (a.D == 128) return launch_attention_d<128>(a, split, stream);
     return launch_attention_d<64>(a, split, stream);
 }

@@ -204,7 +204,6 @@ struct AttnArgs {
     int L, Lc;              // attended positions are clamped to [0, L); Lc = cache axis, multiple of 64
     int cps, ns;            // chunks of 64 positions per split; splits = ceil(Lc / 64 / cps)
     float cs;               // log2(e) * softmax scale
-    uint32_t qflip;         // set by launch_attention: sign bits flipped in q (a negative scale; cs is then its size)
     // Decode (T = 1) with the rotary embedding and the KV-cache append fused in
     // (qkv set; q unused): the q heads and the step's k and v come from the qkv
     // projection output, rotated as w4a8_rope_kv rotates them.

@@ -175,6 +175,32 @@ def test_huge_scores(pkg, dev, D, q_scale, scale):
     check(got, ref, mag, "rotary")
 
 
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("gap", [125, 126, 127, 130])
+def test_probabilities_below_the_normal_range(pkg, dev, gap, first):
+    """A key 2^gap times heavier than all others, whose value is 0 while theirs are 2^118:
+    probabilities (the heavy key in the first chunk) and rescale factors (in the last) below
+    2^-126 keep their subnormal values.  Bound per other key: half a bf16 subnormal step, 2^-134,
+    of its value, beside check()'s."""
+    L, D = 192, 128
+    say(f"attention gap 2^{gap}, heavy key {'first' if first else 'last'}")
+    q = torch.zeros((1, 1, 2, D), dtype=torch.bfloat16, device=dev)
+    k = torch.zeros((1, 1, L, D), dtype=torch.bfloat16, device=dev)
+    vt = torch.full((1, 1, D, L), 2.0 ** 118, dtype=torch.bfloat16, device=dev)
+    heavy = 0 if first else L - 1
+    q[..., 0], k[0, 0, heavy, 0], vt[..., heavy] = 1.0, float(gap), 0.0
+    scale = math.log(2.0)                    # times log2(e): scores are powers of two's exponents
+    p = torch.full((1,), L - 1, dtype=torch.int64, device=dev)
+    ref, mag = reference(q, k, vt, L - 1, L, scale)
+    bound = 2.0 ** -8 * mag + bf16_ulp(ref) + L * 2.0 ** (118 - 134)
+    for cps in (1, 3):
+        for split in (False, True):
+            got = attn(q, k, vt, p, L, cps, split, scale).double().cpu()
+            say(f"  cps={cps} split={split}: {got.flatten()[0].item():.4g}, exactly {ref.flatten()[0].item():.4g}")
+            assert torch.all((got - ref).abs() <= bound)
+            assert torch.all(got > 0)
+
+
 @pytest.mark.parametrize("B,T,H,KVH,D,scale,note", [
     (8, 181, 40, 8, 128, None, "two row tiles per wave, a ragged last workgroup"),
     (8, 181, 40, 8, 64, -0.2, "the same at D = 64, a negative scale"),

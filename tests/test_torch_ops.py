@@ -49,6 +49,47 @@ def test_strided_inputs(pkg, dev, M):
     assert torch.ops.npu.w4a8_linear(x[:0], w, s, N, K, G).shape == (0, N)
 
 
+def _row_views(row):
+    """One row [1, K] under the row strides torch counts as contiguous: K, 1, 0 and an odd one."""
+    K = row.numel()
+    wide = torch.zeros((2, K + 3), dtype=row.dtype, device=row.device)
+    wide[0, :K] = row
+    views = {"K": row.reshape(1, K), "1": row.reshape(K, 1).t(), "0": row.reshape(K).expand(4, K)[:1],
+             "odd": wide[:1, :K]}
+    assert [v.stride(0) for v in views.values()] == [K, 1, 0, K + 3]
+    assert all(v.is_contiguous() for v in views.values())
+    return views
+
+
+def test_rows_pass_through_by_their_strides(pkg):
+    """Only contiguous rows K apart pass through; every other view comes out that way."""
+    x = torch.randn((3, 64)).to(torch.bfloat16)
+    rows = pkg.linear.__globals__["_rows"]
+    assert rows(x) is x
+    cases = list(_row_views(x[0]).values()) + [x.t().contiguous().t(), x.float(), x.view(1, 3, 64), x[:, :32], x[:0]]
+    for v in cases:
+        got = rows(v)
+        assert got.dtype is torch.bfloat16 and got.stride() == (v.shape[-1], 1) and got.is_contiguous()
+        assert torch.equal(got, v.reshape(-1, v.shape[-1]).to(torch.bfloat16))
+
+
+@pytest.mark.gpu
+def test_one_row_strides(pkg, dev):
+    """A single token under every row stride torch counts as contiguous, through each caller."""
+    N, K, G = 256, 1024, 128
+    w, s = _weight(dev, N, K, G, 3)
+    lin = torch.nn.Linear(K, N, bias=True, device=dev)
+    modules = [pkg.W4A8Linear.from_float(lin, G), pkg.MidGroupW4A8Linear.from_float(lin, 512)]
+    mid = modules[1]
+    calls = [lambda x: pkg.linear(x, w, s, N, G), lambda x: pkg.linear_swiglu(x, w, s, N, G), *modules,
+             lambda x: pkg.midgroup_linear(x, mid.weight_packed, *mid._gn, 512)]
+    views = _row_views(torch.randn((1, K), device=dev).to(torch.bfloat16))
+    for i, call in enumerate(calls):
+        want = call(views["K"])
+        for name, v in views.items():
+            assert torch.equal(call(v), want), (i, name)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,G", [
     (1, 5120, 1024, 128),      # fused single row, staged decode plans

@@ -23,8 +23,11 @@ from .packing import quantize_weight
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
-    """x as contiguous bf16 rows [M, K]; an activation that already is one passes through."""
-    if x.dim() == 2 and x.dtype is torch.bfloat16 and x.is_contiguous():
+    """x as contiguous bf16 rows [M, K]; an activation that already is one passes through.
+
+    (By its strides: is_contiguous() ignores a single row's, and the kernels take the row
+    stride as it is -- an expanded or transposed row would have one below K.)"""
+    if x.dim() == 2 and x.dtype is torch.bfloat16 and x.stride() == (x.shape[1], 1):
         return x
     return x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
 

@@ -148,6 +148,35 @@ def test_linear_bias_left_to_torch(pkg, dev):
         torch.testing.assert_close(torch.ops.npu.w4a8_linear(x, w, s, N, K, G, v), y + v, rtol=0, atol=0, equal_nan=True)
 
 
+def test_which_biases_the_op_adds(pkg):
+    """Plain bf16 [N] tensors; none that autograd, forward mode or a function transform (vmap:
+    one GEMM for all biases) has to see."""
+    import torch.autograd.forward_ad as fwd
+    takes = pkg.linear.__globals__["_epilogue_bias"]
+    x, b = torch.zeros((2, 8), dtype=torch.bfloat16), torch.zeros((4,), dtype=torch.bfloat16)
+    seen = []
+
+    def record(t):
+        seen.append(takes(t, x, 4))
+        return (t * 1).sum()
+
+    assert takes(b, x, 4) and takes(torch.nn.Parameter(b, requires_grad=False), x, 4)
+    assert not takes(b.float(), x, 4) and not takes(b[:1], x, 4) and not takes(b.view(1, 4), x, 4)
+    trained = b.clone().requires_grad_()
+    assert not takes(trained, x, 4)
+    with torch.no_grad():
+        assert takes(trained, x, 4)
+    with fwd.dual_level():
+        assert not takes(fwd.make_dual(b, b), x, 4)
+    torch.func.vmap(record)(torch.stack([b, b]))
+    torch.func.vmap(torch.func.grad(record))(torch.stack([b, b]))
+    torch.func.grad(record)(b)
+    torch.func.jvp(record, (b,), (b,))
+    with torch.no_grad():
+        torch.func.vmap(record)(torch.stack([b, b]))
+    assert seen == [False] * 5
+
+
 @pytest.mark.gpu
 def test_bad_inputs_raise(pkg, dev):
     N, K, G = 256, 1024, 128

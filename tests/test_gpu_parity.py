@@ -159,6 +159,28 @@ def test_quant_ties_zero_rows_and_strided_input(dev):
     assert torch.equal(a_q2, a_q) and torch.equal(a_s2, a_s)
 
 
+@pytest.mark.parametrize("e", [120, 20, 0, -60, -92, -94, -110])
+def test_quant_every_significand(pkg, dev, e):
+    """A row per significand of the absmax (so of nearly every scale significand), holding every
+    bf16 value of both signs from the absmax down ten octaves: all half-way quotients there are,
+    at scales through the range of the reciprocal, at its 2^-100 end and below it (divides)."""
+    say(f"quant every significand, absmax 2^{e}")
+    mant = (1 + np.arange(128) / 128.0)
+    amax = mant * 2.0 ** e
+    cols = np.concatenate([np.outer(2.0 ** -np.arange(1, 11, dtype=np.float64), mant).reshape(-1)])
+    x = np.minimum(cols[None, :] * 2.0 ** e * 2, np.inf)       # 2^e .. down
+    x = np.where(x <= amax[:, None], x, amax[:, None])
+    x = np.concatenate([amax[:, None].repeat(8, 1), x, -x], 1).astype(np.float32)
+    xb = ow.f32_to_bf16_bits(x)
+    assert np.array_equal(ow.bf16_bits_to_f32(xb), x)
+    a_q, a_s = torch.ops.npu.w4a8_quant_pertoken(bf16_bits_tensor(xb).to(dev))
+    q_ref, s_ref = ow.quant_act_per_token(xb)
+    assert np.array_equal(tensor_bf16_bits(a_s), s_ref)
+    assert np.array_equal(a_q.cpu().numpy(), q_ref)
+    quot = x.astype(np.float64) / ow.bf16_bits_to_f32(s_ref)[:, None].astype(np.float64)
+    assert np.count_nonzero(np.abs(quot - np.trunc(quot)) == 0.5) > 100
+
+
 @pytest.mark.parametrize("K", [512, 27648])
 def test_quant_tiny_and_boundary_scales(pkg, dev, K):
     """Rows whose scale is subnormal, at the 2^-125 edge of the reciprocal path,

@@ -165,6 +165,38 @@ def test_reciprocal_quant_equals_divide_exhaustively():
     assert np.array_equal(reciprocal_quant(ow.bf16_bits_to_f32(xb), sf), q)
 
 
+def refined_quant(xf: np.ndarray, s: np.float32) -> np.ndarray:
+    """numpy model of the GPU quantiser's arithmetic for a scale s >= 2^-100: q0 = fp32(x *
+    fp32(1/s)), q = q0 + (x - q0 s) / s by two fused multiply-adds (float64 holds both products
+    exactly), then the fp32 sum with 1.5 * 2^23."""
+    r = np.float32(1.0) / s
+    q0 = xf * r
+    e = (xf.astype(np.float64) - q0.astype(np.float64) * np.float64(s)).astype(np.float32)
+    q = (q0.astype(np.float64) + e.astype(np.float64) * np.float64(r)).astype(np.float32)
+    u = np.minimum(q + np.float32(12582912.0), np.float32(12582912.0 + 127.0))
+    return (u.view(np.uint32) & 0xff).astype(np.uint8).view(np.int8)
+
+
+def test_refined_quant_equals_divide_exhaustively():
+    """The refined reciprocal gives the IEEE divide's codes for every bf16 x with |x| <=
+    127.25 s and every bf16 significand of s, at the largest, two middle and the smallest
+    scale exponents it is used for."""
+    allx = ow.bf16_bits_to_f32(np.arange(0, 1 << 16, dtype=np.uint32).astype(np.uint16))
+    allx = allx[np.isfinite(allx)]
+    ties = 0
+    for e in (126, 20, -40, -100):
+        for m in range(128, 256):
+            s = np.float32(m * 2.0 ** (e - 7))
+            if s > 3.0e38:
+                continue
+            x = allx[np.abs(allx.astype(np.float64)) <= 127.25 * np.float64(s)]
+            q = (x / s).astype(np.float32)
+            div = np.clip(np.rint(q), -128, 127).astype(np.int8)
+            assert np.array_equal(refined_quant(x, s), div), (e, m)
+            ties += int(np.count_nonzero(np.abs(q - np.trunc(q)) == 0.5))
+    assert ties > 1000
+
+
 # --------------------------------------------------------------- packing / geometry
 RAGGED_CASES = [(5120, 128), (27648, 128), (1057, 128), (1279, 256), (1025, 1024), (33, 64), (1, 64), (65, 64),
                 (63, 64), (2049, 512), (1023, 1024), (35, 32), (777, 96), (100, 33), (4096, 64)]

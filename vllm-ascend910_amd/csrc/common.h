@@ -150,43 +150,26 @@ __device__ __forceinline__ int quant_div(float x, float s) {
     return static_cast<int>(q);
 }
 
-// The row's scale, its reciprocal and half of it.  With s normal (>= 2^-125
-// here) and |x| <= 127.25 s (s = bf16(amax / 127) is at least amax / 127
-// less one bf16 rounding), y = x * (1/s) lies within 2^-16 of the exact x/s,
-// and x/s -- a ratio of two 8-bit significands -- is either a half-integer or
-// at least 2^-10 from every half-integer.  So rint(y) is rint(x/s) except at
-// exact half-way cases, where the residual x - t*s (exact in an fma) is
-// +-s/2 and the even neighbour is taken.  Other scales (subnormal, infinite,
-// NaN) divide per element.
+// The row's scale and its reciprocal.  fast: the quotients of the row's elements
+// come from the reciprocal (quant8_fast); other scales (2^-100 and below,
+// infinite, NaN) divide per element.
 struct RowScale {
-    float s, r, hs;
+    float s, r;
     bool fast;
 };
 
 __device__ __forceinline__ RowScale row_scale(float s) {
     RowScale q;
     q.s = s;
-    q.fast = s >= 0x1p-125f && s <= 3.0e38f;
+    q.fast = s >= 0x1p-100f && s <= 3.0e38f;
     q.r = 1.0f / s;
-    q.hs = 0.5f * s;
     return q;
 }
 
-template <bool FAST>
-__device__ __forceinline__ int quant_code(float x, const RowScale& q) {
-    if constexpr (!FAST) return quant_div(x, q.s);
-    const float t = rintf(x * q.r);
-    const float d = fmaf(-t, q.s, x);
-    int v = static_cast<int>(t);
-    if (fabsf(d) == q.hs && (v & 1)) v += d > 0.0f ? 1 : -1;
-    return min(127, max(-128, v));
-}
-
 // Cross-lane steps of a wave in the vector pipe (DPP and the gfx950 lane swaps;
-// a __shfl_xor is an LDS permute the wave waits for).  xor_lane<B>(v): the value
-// of lane ^ (1 << B).  Bits 2 and 3 are mirrors of 8 and 16 lanes, which reach a
-// lane ^ 4 (^ 8) only where the lanes below that bit already agree: use them in
-// increasing order of B, as the reductions below do.
+// a __shfl_xor is an LDS permute the wave waits for): an xor butterfly over lane
+// bits 0, 1, ... 5.  Bits 2 and 3 are mirrors of 8 and 16 lanes, which reach lane
+// ^ 4 (^ 8) only because the lanes below that bit already agree.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_mov(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xf, 0xf, true));
@@ -216,32 +199,30 @@ __device__ __forceinline__ int wave_sum(int v) {
     return static_cast<int>(wave_reduce(static_cast<uint32_t>(v), [](uint32_t a, uint32_t b) { return a + b; }));
 }
 
-// Two bf16 in one dword -> two int8 codes in the low 16 bits.
-template <bool FAST>
-__device__ __forceinline__ uint32_t quant2(uint32_t u, const RowScale& q) {
-    const int q0 = quant_code<FAST>(__uint_as_float(u << 16), q);
-    const int q1 = quant_code<FAST>(__uint_as_float(u & 0xffff0000u), q);
-    return (static_cast<uint32_t>(q0) & 0xffu) | ((static_cast<uint32_t>(q1) & 0xffu) << 8);
-}
-
-// Eight bf16 -> eight int8 codes (a RowScale with fast set).  x * r + 1.5 * 2^23 in
-// one fused multiply-add rounds x * r to its nearest integer and leaves it in the
-// low byte; as in RowScale, that is rint(x / s) except at an exact half-way
-// quotient, where |x - t s| = s / 2: `tie` is then set, and the caller takes
-// quant8 for the wave (about one wave in forty on random rows).  Five vector
-// instructions per element and no per-element select, against about fourteen
-// for quant_code: the single-row linear of K = 27648 quantises 54 elements per
-// lane before its first product.
+// Eight bf16 -> eight int8 codes (a RowScale with fast set): rint of the quotient
+// by one rounded addition of 1.5 * 2^23, which leaves it in the low byte.  The
+// quotient is x * r refined once, q = q0 + (x - q0 s) r with two fused
+// multiply-adds.  x/s, a ratio of two 8-bit significands with |x| <= 127.25 s
+// (s = bf16(amax / 127) is at least amax / 127 less one bf16 rounding), is either
+// a half-integer or at least 2^-10 from every half-integer.  Away from one, q is
+// within 2^-16 of x/s.  At a half-integer h, h - q0 is a few units in the last
+// place of q0, so x - q0 s = (h - q0) s is exact (s >= 2^-100 keeps it a float)
+// and q0 + (h - q0) s r rounds to h itself: ties go to even as in the divide.
+//
+// Six vector instructions per element and no tie to look for.  A test for ties and
+// a second code sequence for the waves that hold one (one in forty on random rows)
+// was as short, but a call waits for its slowest wave, and the rare sequence is
+// cold in the instruction cache: quant of 64 rows of 27648 4.9 -> 3.7 us, of one
+// row of 5120 3.2 -> 2.5, RMSNorm + quant of 64 rows of 8192 5.2 -> 3.8.
 constexpr float kRoundMagic = 12582912.0f;
-__device__ __forceinline__ uint2 quant8_fast(const uint4& v, const RowScale& q, bool& tie) {
+__device__ __forceinline__ uint2 quant8_fast(const uint4& v, const RowScale& q) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
     uint32_t c[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const float x = __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
-        const float u = fmaf(x, q.r, kRoundMagic);
-        const float d = fmaf(kRoundMagic - u, q.s, x);
-        tie = tie || fabsf(d) == q.hs;
+        const float q0 = x * q.r;
+        const float u = fmaf(fmaf(-q0, q.s, x), q.r, q0) + kRoundMagic;
         c[j] = __float_as_uint(fminf(u, kRoundMagic + 127.0f));
     }
     uint32_t o[2];
@@ -252,23 +233,26 @@ __device__ __forceinline__ uint2 quant8_fast(const uint4& v, const RowScale& q, 
     return make_uint2(o[0], o[1]);
 }
 
-// The same codes element by element, for every RowScale.
-template <bool FAST>
-__device__ __forceinline__ uint2 quant8(const uint4& v, const RowScale& q) {
-    return make_uint2(quant2<FAST>(v.x, q) | (quant2<FAST>(v.y, q) << 16),
-                      quant2<FAST>(v.z, q) | (quant2<FAST>(v.w, q) << 16));
+// The same codes by a divide per element, for every scale.
+__device__ __forceinline__ uint2 quant8_div(const uint4& v, const RowScale& q) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t o[2] = {0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float x = __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
+        o[j >> 2] |= (static_cast<uint32_t>(quant_div(x, q.s)) & 0xffu) << (8 * (j & 3));
+    }
+    return make_uint2(o[0], o[1]);
 }
 
-// The codes of one 16-byte unit per lane.  One wave-uniform branch to the element
-// by element forms (on a ballot: a condition the compiler takes for per-lane is
-// turned into selects, and the divides then run for every row).
+// The codes of one 16-byte unit per lane.  One wave-uniform branch to the divides
+// (on a ballot: a condition the compiler takes for per-lane is turned into
+// selects, and the divides then run for every row), after the fast form: put
+// before it, the divides stood in the way of the instruction fetch (64 rows of
+// 27648 3.7 -> 4.5 us, one row of RMSNorm + quant of 5120 3.2 -> 3.9).
 __device__ __forceinline__ uint2 quant_unit(const uint4& v, const RowScale& q) {
-    bool slow = !q.fast;
-    uint2 o = quant8_fast(v, q, slow);
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(slow) != 0, 0)) {
-        if (__builtin_amdgcn_ballot_w64(!q.fast) != 0) o = quant8<false>(v, q);
-        else o = quant8<true>(v, q);
-    }
+    uint2 o = quant8_fast(v, q);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!q.fast) != 0, 0)) o = quant8_div(v, q);
     return o;
 }
 

@@ -8,9 +8,9 @@
 // The quotient is the IEEE divide's (the reference kernel insists on it,
 // npu_ops/kernel/midgroup_quant_a.inc:55-62): a plain reciprocal multiply
 // would flip half-way cases relative to torch.  The codes here come from a
-// reciprocal multiply plus an exact half-way test (RowScale, quant_unit, common.h) that gives
-// the divide's result for every input; rows whose scale is not a normal
-// float divide per element.
+// reciprocal multiply refined once (quant8_fast, common.h), which gives the
+// divide's result for every input; rows whose scale is tiny, infinite or NaN
+// divide per element.
 //
 // Layout: one workgroup per row (256 threads, 1024 for rows longer than 8192
 // elements, so a decode-sized call still has enough loads in flight; long
@@ -83,7 +83,7 @@ __device__ __forceinline__ void zero_pads(int8_t* qr, int K, const PadMap& pm) {
 // (SPLIT only) are read in a loop instead, and the workgroup's own units again.
 //
 // Bound by memory on many rows (16384 x 27648: 259 -> 231 us, 5.9 TB/s of its 1.36
-// GB, from five instead of fourteen vector instructions per element) and by
+// GB, from six instead of fourteen vector instructions per element) and by
 // latency on few: one memory round trip, two block-wide steps and the per-element
 // work of a thread's units (1 x 5120 3.1 -> 2.6 us in a graph of back-to-back calls).
 template <int VPT, int NT, bool PAD, bool SPLIT>
@@ -145,11 +145,11 @@ __global__ __launch_bounds__(kThreads) void quant_act_scalar_kernel(
     for (int k = threadIdx.x; k < K; k += kThreads) amax = max(amax, static_cast<uint32_t>(xr[k]) & 0x7fffu);
     amax = block_max<kThreads>(amax, red);
     const uint32_t sbits = scale_from_amax(amax);
-    const RowScale q = row_scale(bf16_bits_to_f32(sbits));
+    const float s = bf16_bits_to_f32(sbits);
     if (threadIdx.x == 0) ascale[row] = static_cast<uint16_t>(sbits);
     int8_t* qr = aq + row * lda;
     for (int k = threadIdx.x; k < K; k += kThreads)
-        qr[pad ? pad_dst(k, pm) : k] = static_cast<int8_t>(quant_code<false>(bf16_bits_to_f32(xr[k]), q));
+        qr[pad ? pad_dst(k, pm) : k] = static_cast<int8_t>(quant_div(bf16_bits_to_f32(xr[k]), s));
     if (pad) zero_pads<1>(qr, K, pm);
 }
 

@@ -22,7 +22,7 @@
 // later slots twice.  A two-pass form with 2-byte loads and an IEEE divide
 // per element took 261 us at 4096 x 27648 (this one 85).
 // The quotient rint(x / s) is taken in the reciprocal form of common.h
-// (row_scale / quant_code), equal to the IEEE divide for these scales.
+// (quant_unit), equal to the IEEE divide for these scales.
 #include "common.h"
 #include "kgeom.h"
 #include "launch.h"

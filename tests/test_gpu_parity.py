@@ -1661,6 +1661,23 @@ def test_rmsnorm_quant_rows_do_not_depend_on_batch(pkg, dev, K):
             assert torch.equal(t65[:1].view(torch.int8).cpu(), t1.view(torch.int8).cpu()), "row 0 differs, M=1 vs 65"
 
 
+@pytest.mark.parametrize("M", [1, 65])
+@pytest.mark.parametrize("K", [264, 4096, 5120, 12288, 16392, 32776])
+def test_rmsnorm_quant_infinite_normed_rows(pkg, dev, M, K):
+    """eps = 0 and squares that underflow: 1 / rms is infinite and so is every normed value.
+    The row's scale is infinite (not NaN), whether or not the row fills its workgroup's units."""
+    say(f"rmsnorm_quant infinite M={M} K={K}")
+    x = torch.full((M, K), 1e-24, dtype=torch.bfloat16, device=dev)
+    x[:, ::3] *= -1
+    w = torch.ones((K,), dtype=torch.bfloat16, device=dev)
+    for res in (None, torch.zeros_like(x)):
+        a_q, a_s, _, h = torch.ops.npu.w4a8_rmsnorm_quant(x, w, 0.0, res, 0, True)
+        assert torch.equal(h, torch.where(x > 0, float("inf"), float("-inf")).to(torch.bfloat16))
+        assert torch.all(torch.isposinf(a_s))
+        q_ref, s_ref = torch.ops.npu.w4a8_quant_pertoken(h)
+        assert torch.equal(a_q, q_ref) and torch.equal(a_s, s_ref)
+
+
 # ------------------------------------------------------------------ checkpoint formats
 def test_vendor_checkpoint_linear(pkg, dev):
     """A vendor W4A8_DYNAMIC linear (packed along N, per-channel x per-group scales) loaded

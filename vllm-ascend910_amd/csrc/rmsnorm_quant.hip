@@ -150,7 +150,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     for (int i = 0; i < VPT; ++i) {
         const int idx = static_cast<int>(threadIdx.x) + i * NT;
         if (p.sum_out && idx < nvec) *reinterpret_cast<uint4*>(p.sum_out + row * p.lds + idx * 8) = v[i];
-        // (units past the row: zeros times a zero weight)
+        // (units past the row: zeros times a zero weight, NaN where r is infinite)
         uint32_t* pa = reinterpret_cast<uint32_t*>(&v[i]);
         const uint32_t* pw = reinterpret_cast<const uint32_t*>(&wv[i]);
 #pragma unroll
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
             pa[d] = f32x2_to_bf16x2_bits(__uint_as_float(n << 16) * __uint_as_float(pw[d] << 16),
                                          __uint_as_float(n & 0xffff0000u) * __uint_as_float(pw[d] & 0xffff0000u));
         }
-        amax = max(amax, abs_bits_max8(v[i]));
+        if (idx < nvec) amax = max(amax, abs_bits_max8(v[i]));
         if (p.h_out && idx < nvec) *reinterpret_cast<uint4*>(p.h_out + row * p.ldh + idx * 8) = v[i];
     }
     amax = block_max_u<NT>(amax, redu);

@@ -93,6 +93,15 @@ __device__ __forceinline__ uint32_t block_max_u(uint32_t v, uint32_t* red) {
 
 
 // VPT units of 8 elements per thread; K % 8 == 0, rows 16-byte aligned.
+//
+// Bound by latency on few rows (the row's load, two block-wide reductions and the
+// per-element work in between) and by memory on many (2048 x 5120 with the residual:
+// 16 us, 4.8 TB/s of its 79 MB).  Two things keep the long rows (1024 threads) from
+// more: waves whose unit lies past the row skip its work, and at eight units per
+// thread the weight is loaded after the reduction, where row, residual and weight
+// together would spill (2048 rows of 32776: 390 us with both left out, 152 now; 64
+// rows of 5120 on 640 of 1024 threads 3.8 -> 3.5).  The 256-thread forms do not
+// skip: full rows of 8192 lose more (256 rows 4.2 -> 4.5 us) than tails gain.
 template <int VPT, int NT, bool RES>
 __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     static_assert((VPT & (VPT - 1)) == 0 && (NT & (NT - 1)) == 0, "power-of-two units and threads");
@@ -101,8 +110,9 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     const int64_t row = blockIdx.x;
     const int nvec = p.K >> 3;
     // Buffer loads (units past the row read zero), all requested before the first
-    // is used: the row, the residual, and the norm weight (used after the
-    // reduction, which would otherwise wait for a second memory round trip).
+    // is used: the row, the residual, and (up to four units) the norm weight, used
+    // after the reduction, which would otherwise wait for a second memory round trip.
+    constexpr bool kEarlyW = VPT < 8, kSkip = NT == 1024;
     const uint32_t bytes = static_cast<uint32_t>(p.K) * 2u;
     const auto xr = make_rsrc(p.x + row * p.ldx, bytes);
     const auto rr = make_rsrc(RES ? p.res + row * p.ldr : p.x, RES ? bytes : 0u);
@@ -114,8 +124,14 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
         xv[i] = buf_load16(xr, o);
         if constexpr (RES) rv[i] = buf_load16(rr, o);
     }
+    auto load_w = [&](int i) { return buf_load16(wr, (threadIdx.x + static_cast<uint32_t>(i * NT)) * 16u); };
+    if constexpr (kEarlyW) {
 #pragma unroll
-    for (int i = 0; i < VPT; ++i) wv[i] = buf_load16(wr, (threadIdx.x + static_cast<uint32_t>(i * NT)) * 16u);
+        for (int i = 0; i < VPT; ++i) wv[i] = load_w(i);
+    }
+    // unit i holds a part of the row somewhere in this wave (wave-uniform)
+    const int wave0 = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x & ~63u));
+    auto live = [&](int i) { return !kSkip || wave0 + i * NT < nvec; };
     // s = bf16(x + r) kept as packed bf16 pairs; per-thread sum of squares
     uint4 v[VPT];
     float ss[VPT];
@@ -143,11 +159,16 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     }
     const float tot = block_sum_units<VPT, NT>(ss, redf);
     const float r = 1.0f / sqrtf(tot / static_cast<float>(p.K) + p.eps);
+    if constexpr (!kEarlyW) {
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) wv[i] = load_w(i);
+    }
 
     // h = bf16(bf16(s * r) * w); absmax of h
     uint32_t amax = 0u;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
+        if (!live(i)) continue;
         const int idx = static_cast<int>(threadIdx.x) + i * NT;
         if (p.sum_out && idx < nvec) *reinterpret_cast<uint4*>(p.sum_out + row * p.lds + idx * 8) = v[i];
         // (units past the row: zeros times a zero weight, NaN where r is infinite)
@@ -171,6 +192,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_kernel(const RmsParams p) {
     int8_t* qr = p.a_q + row * p.lda;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
+        if (!live(i)) continue;
         const int idx = static_cast<int>(threadIdx.x) + i * NT;
         const uint2 o = quant_unit(v[i], sc);
         if (idx >= nvec) continue;

@@ -143,6 +143,21 @@ def test_quant_split_rows_mixed_ties(dev, M, K, group):
     assert np.array_equal(a_q.cpu().numpy()[rows], ow.pad_groups(q_ref, group) if group else q_ref)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17])
+@pytest.mark.parametrize("K", [32776, 65536, 65544, 139272])
+def test_quant_rows_past_the_registers(pkg, dev, M, K):
+    """Rows longer than a workgroup holds: the last length held by eight units of 1024 threads
+    (65536), the next one, and two passes of the absmax loop with a part of a unit left; the
+    absmax in the row's last element, which only one thread of one workgroup quantises."""
+    say(f"quant long rows M={M} K={K}")
+    xb = pkg.synth.activations(M, K, seed=K + M)
+    xb[:, -1] = ow.f32_to_bf16_bits(np.float32(-700.0))
+    a_q, a_s = torch.ops.npu.w4a8_quant_pertoken(bf16_bits_tensor(xb).to(dev))
+    q_ref, s_ref = ow.quant_act_per_token(xb)
+    assert np.array_equal(tensor_bf16_bits(a_s), s_ref)
+    assert np.array_equal(a_q.cpu().numpy(), q_ref)
+
+
 def test_quant_ties_zero_rows_and_strided_input(dev):
     say("quant ties/zero/strided")
     xb = tie_rows(64, 512, seed=11)

@@ -101,8 +101,17 @@ __global__ __launch_bounds__(NT) void quant_act_vec_kernel(
     uint4 v[VPT];
     uint32_t amax = 0u;
     if (SPLIT && static_cast<int>(gridDim.y) > VPT) {
-        for (int i = 0; i < static_cast<int>(gridDim.y); ++i) amax = max(amax, abs_bits_max8(unit(i)));
-        v[0] = unit(own);
+        // eight loads in flight for a few rows (VPT = 8); one at a time past 16 rows, where
+        // the workgroups of a CU hide each other's latency (40960 x 64 rows 4.8 us against 5.4)
+        constexpr int U = VPT == 8 ? 8 : 1;
+        const uint4 w = unit(own);
+        for (int i0 = 0; i0 < static_cast<int>(gridDim.y); i0 += U) {
+#pragma unroll
+            for (int i = 0; i < U; ++i) v[i] = unit(i0 + i);
+#pragma unroll
+            for (int i = 0; i < U; ++i) amax = max(amax, abs_bits_max8(v[i]));
+        }
+        v[0] = w;
     } else {
 #pragma unroll
         for (int i = 0; i < VPT; ++i) v[i] = unit(i);
@@ -176,16 +185,19 @@ hipError_t launch_quant_act(const uint16_t* x, int64_t ldx, int8_t* a_q, int64_t
     // Rows of up to 8192 elements: 256 threads.  Longer rows of a small batch
     // (M < 256, too few rows to fill the GPU) are split: over 512-thread workgroups
     // of one 16-byte unit per thread up to 16 rows, 1024-thread ones past them
-    // (K = 27648, us: 16 rows 3.7 / 4.0, 64 rows 5.2 / 4.8, 200 rows 9.5 / 8.7).
+    // (K = 27648, us: 16 rows 3.2 / 3.3, 64 rows 4.1 / 3.7, 200 rows 7.2 / 6.8) and for
+    // rows past 32768 elements, which 512 threads no longer hold (131072: one row
+    // 6.9 us / 4.7, 16 rows 7.5 / 5.5, each against the better loop).
     // Longer rows otherwise: 1024 threads per row.
     const bool vec = aligned && K < (int64_t{1} << 30);   // rows in 32-bit buffer offsets
     if (vec && nvec > 4 * kThreads && M < 256) {
-        const int nt = M <= 16 ? 512 : 1024;
+        const int nt = M <= 16 && nvec <= 8 * 512 ? 512 : 1024;
         const dim3 g2(static_cast<unsigned>(M), static_cast<unsigned>((nvec + nt - 1) / nt));
 #define W4A8_QSPLIT(V, NT)                                                                                     \
     if (pad) quant_act_vec_kernel<V, NT, true, true><<<g2, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm); \
     else quant_act_vec_kernel<V, NT, false, true><<<g2, dim3(NT), 0, stream>>>(x, ldx, a_q, lda, a_scale, iK, pm);
         if (nt == 512) { W4A8_QSPLIT(8, 512) }
+        else if (M <= 16) { W4A8_QSPLIT(8, 1024) }
         else { W4A8_QSPLIT(4, 1024) }
 #undef W4A8_QSPLIT
         return hipGetLastError();

@@ -158,6 +158,19 @@ def test_rope_kv_prefill_layout(pkg, dev, B, T, H, KVH, D, L, p0, with_bias):
     assert bits_equal(q[:, t0:t1], q_ref) and bits_equal(k_view, kc_ref) and bits_equal(v_view, vc_ref)
 
 
+@pytest.mark.parametrize("B,T,H,KVH,D,L,p0,with_bias", [
+    (1, 319, 12, 2, 64, 320, 0, True),     # at 256 CUs the most (token, head) pairs of the other kernel
+    (5, 64, 12, 2, 64, 64, 0, True),       # the fewest of this one
+    (40, 65, 4, 2, 64, 70, 5, False),      # a v tile and one token, an odd offset
+    (4, 150, 10, 2, 128, 192, 42, True),   # up to the last cache position
+    (8, 70, 6, 3, 96, 90, 30, True),       # ten tokens past the cache end, D = 96
+    (24, 33, 4, 2, 64, 64, -3, False),     # three tokens before position 0
+])
+def test_rope_kv_prefill_layout_by_pairs(pkg, dev, B, T, H, KVH, D, L, p0, with_bias):
+    """The same around the number of (token, head) pairs from which the prefill kernel is taken."""
+    test_rope_kv_prefill_layout(pkg, dev, B, T, H, KVH, D, L, p0, with_bias)
+
+
 def test_rope_kv_graph_replays_follow_the_position(pkg, dev):
     """Captured once; each replay reads the position from the device and the step advances it."""
     B, H, KVH, D, L = 2, 40, 8, 128, 32

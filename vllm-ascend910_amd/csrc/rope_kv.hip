@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64) void rope_kv_kernel(const RopeKvArgs a) {
 // pairs per thread with 16-byte loads and stores, and the others take 64 tokens
 // of one v head through LDS, so every store covers consecutive positions.  The
 // same operations per element, so the same bits.  Bound by memory: 1024 tokens of
-// 40 + 16 heads of 128 (29 MB) 26.1 -> 8.8 us.
+// 40 + 16 heads of 128 (29 MB) 26.1 -> 8.8 us,
 // 8 sequences of them 167 -> 40.
 constexpr int kRopeTile = 64;   // tokens per v workgroup
 
@@ -185,13 +185,17 @@ bool prefill_layout(const RopeKvArgs& a) {
 hipError_t launch_rope_kv(const RopeKvArgs& a, hipStream_t stream) {
     const int64_t tokens = static_cast<int64_t>(a.B) * a.T;
     if (tokens <= 0) return hipSuccess;
-    // From 128 tokens on, a quarter of a v tile or more per sequence (us, the kernel above /
-    // this one: 1 x 64 tokens 4.0 / 4.5, 8 x 16 5.6 / 4.2, 1 x 256 8.5 / 5.2); a decode
-    // step has one token per sequence.
+    // The kernel above is one wave per (token, head).  Up to about twenty waves a CU they
+    // are all resident and it is the quicker; past that, with a quarter of a v tile or more
+    // per sequence, the prefill kernel (us, above / this one: 40 + 16 heads x 64 tokens
+    // 4.2 / 4.5, x 128 5.6 / 5.0, x 256 8.5 / 5.2; 10 + 4 heads x 128 tokens 3.7 / 4.5, x 256
+    // 4.3 / 4.7, x 400 5.2 / 4.7; 32 + 16 heads of 64 x 80 tokens 4.3 / 3.9).  A decode step
+    // has one token per sequence.
+    const int64_t waves = tokens * (a.H + 2 * a.KVH);
     const int tiles = (a.T + kRopeTile - 1) / kRopeTile;
     const int64_t nqk = (tokens * (a.H + a.KVH) * (a.D / 16) + 255) / 256;
     const int64_t nwg = nqk + static_cast<int64_t>(a.B) * tiles * a.KVH;
-    if (a.T >= kRopeTile / 4 && tokens >= 2 * kRopeTile && prefill_layout(a) && nwg < (int64_t{1} << 31)) {
+    if (a.T >= kRopeTile / 4 && waves >= 20 * device_cu_count() && prefill_layout(a) && nwg < (int64_t{1} << 31)) {
         const size_t lds = static_cast<size_t>(kRopeTile) * (a.D + 2) * 2;
         rope_kv_prefill_kernel<<<dim3(static_cast<unsigned>(nwg)), dim3(256), lds, stream>>>(
             a, static_cast<int>(nqk), tiles);

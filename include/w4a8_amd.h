@@ -216,9 +216,11 @@ int w4a8_linear(const void* x, int64_t ldx, const void* w_tiles, const void* s_t
 
 /*
  * w4a8_linear with a bias (bf16 [N], 2-byte aligned, or NULL) added to the bf16
- * outputs in the GEMM's epilogue (more than 64 rows, else W4A8_ERR_UNSUPPORTED): y = bf16(bf16(x @ W.T) + bias), the bits of a
+ * outputs in the GEMM's epilogue: y = bf16(bf16(x @ W.T) + bias), the bits of a
  * bf16 tensor add after w4a8_linear (the reference's apply,
- * npu_ops/python/midgroup_quant.py:163-177).
+ * npu_ops/python/midgroup_quant.py:163-177).  Only the prefill kernels have that
+ * epilogue: a bias with 64 rows or fewer is refused (W4A8_ERR_UNSUPPORTED; add it
+ * to w4a8_linear's output there).
  */
 int w4a8_linear_bias(const void* x, int64_t ldx, const void* w_tiles, const void* s_tiles, int scale_dtype,
                      const void* bias, void* y, int64_t ldy, void* a_q, int64_t lda, void* a_scale, int64_t M,

@@ -94,15 +94,6 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2_bits(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
-// A bf16 output plus a bf16 bias element, rounded as torch adds two bf16 tensors.
-// The prefill epilogues add it to outputs they hold anyway (the columns' bias is read
-// into LDS ahead of the K loop): a launch and a pass over y fewer, 1000 x 7168 x 5120
-// with bias 60.2 -> 54.0 us.  The decode kernels do not: the test for a bias alone
-// took calls without one from 7.4 to 7.7 us at 16 rows.
-__device__ __forceinline__ uint32_t add_bias_bits(uint32_t y, uint32_t b) {
-    return f32_to_bf16_bits(bf16_bits_to_f32(y) + bf16_bits_to_f32(b));
-}
-
 // SwiGLU of one gate/up output pair, rounded the way torch evaluates
 // `F.silu(g) * u` on bf16 tensors (the reference's decoder layer,
 // npu_ops/python/bench_decode_layer.py:78-81): g and u are first rounded to the

@@ -500,7 +500,7 @@ constexpr int kSpP(int mt) { return mt == 1 ? 4 : 2; }   // activation steps in 
 template <int MT>
 __global__ __launch_bounds__(64 * kShWaves) void gemm_midgroup_split_kernel(const MidParams p, int32_t* __restrict__ I,
                                                                            int64_t ldi) {
-    constexpr int R = 16 * MT, CPW = kShCPW, D = kShD, P = kSpP(MT);
+    constexpr int CPW = kShCPW, D = kShD, P = kSpP(MT);
     static_assert(D == 4 && (P == 2 || P == 4), "the unrolled step indexes the rings statically");
     // two steps of two tiles, each tile [row block][plane][row][64 B]; thread tid stages
     // the 16 bytes at tid * 16 of every row block's 4 KB

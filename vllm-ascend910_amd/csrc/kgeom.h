@@ -64,4 +64,9 @@ __host__ __device__ constexpr bool is_unpadded(int64_t K, int64_t group) {
 }
 
 }  // namespace geom
+
+// Most rows of the decode GEMMs (their plans hold up to four 16-row tiles); more take
+// the prefill kernels, whose epilogue can add a bias.
+constexpr int64_t kDecodeMaxM = 64;
+
 }  // namespace w4a8

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kgeom.h"
+
 namespace w4a8 {
 
 // group > 0 with a ragged geometry (kpad != K) writes the padded group layout.
@@ -37,9 +39,7 @@ struct GemmArgs {
     int64_t workspace_bytes;
 };
 
-// Decode path (M <= kDecodeMaxM): weight-stream bound, split-K.
-constexpr int64_t kDecodeMaxM = 64;
-
+// Decode path (M <= kDecodeMaxM, kgeom.h): weight-stream bound, split-K.
 int64_t decode_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group);
 hipError_t launch_gemm_decode(const GemmArgs& a, hipStream_t stream);
 

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kThreadsMG) void quant_midgroup_kernel(const MidQua
         sbits[r] = f32_to_bf16_bits(bf16_bits_to_f32(am) / 127.0f);
         if ((sbits[r] & 0x7fffu) == 0u) sbits[r] = kTinyBits;
         if (row >= p.Mp) continue;
-        // q = clamp(rint(x / s)): the reciprocal form with its tie correction
+        // q = clamp(rint(x / s)): the refined reciprocal form
         // (common.h: exact for these scales, |x| <= 127.25 s), else a divide
         const RowScale q = row_scale(bf16_bits_to_f32(sbits[r]));
         const bool live = row < p.M;

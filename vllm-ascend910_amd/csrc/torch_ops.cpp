@@ -204,8 +204,8 @@ Tensor linear(const Tensor& x0, const Tensor& w_tiles, const Tensor& s_tiles, in
     const Tensor aq = empty({as_off + 2 * M}, at::kChar, x);
     char* const p = static_cast<char*>(aq.data_ptr());
     const Abi& f = abi();
-    // the prefill kernels' epilogue adds the bias; up to 64 rows torch does
-    const bool epilogue = bias.has_value() && M > 64;
+    // the prefill kernels' epilogue adds the bias; up to kDecodeMaxM rows torch does
+    const bool epilogue = bias.has_value() && M > w4a8::kDecodeMaxM;
     const int64_t need = f.w4a8_gemm_workspace_bytes(M, N, K, group);
     const Workspace ws = need > 0 ? workspace(x, need) : Workspace{};
     check(f.w4a8_linear_bias(x.data_ptr(), x.stride(0), w_tiles.data_ptr(), s_tiles.data_ptr(), scale_code(s_tiles),

@@ -1362,8 +1362,8 @@ def test_midgroup_prefill_qwq_shapes(pkg, dev, proj, M):
 def test_midgroup_decode_reference_order(pkg, dev, proj, M):
     """Decode rows at group 1024: the K split over waves adds exact int32 group sums and folds
     once in group order (or one wave walks every group), so the output is bf16 of the
-    reference's fp32 result bit for bit -- down_proj past 16 rows included, whose 27 groups
-    of 64-row sums exceed the LDS and which takes 32-row tiles."""
+    reference's fp32 result bit for bit -- down_proj at 16 and 64 rows included, whose K is
+    split over workgroups of one to three groups each."""
     K, N = pkg.synth.QWQ_SHAPES[proj]
     say(f"midgroup decode order {proj} M={M}")
     xb, codes, sc, zr, a, args = _midgroup_inputs(pkg, dev, M, N, K, 1024, True, seed=31 + M)
@@ -1390,7 +1390,7 @@ def _tiles_ref(w_q: np.ndarray, KT: int) -> np.ndarray:
     (1, 7168, 5120, 1024),      # per-wave kernel, int32 group sums
     (16, 1000, 1057, 1024),     # ragged K (a half-padding last tile), N not a multiple of 16
     (1, 16400, 1057, 1024),     # shared-activation kernel on wide N
-    (64, 5120, 27648, 1024),    # 32-row tiles (27 groups of sums)
+    (64, 5120, 27648, 1024),    # K split over workgroups (27 groups over 12 on 256 CUs)
     (48, 2064, 3456, 256),      # 64-row tiles, stride 256
     (300, 8200, 5120, 1024),    # prefill path on the tiles
     (2048, 1000, 1057, 1024),   # prefill path (the stored rows would be repacked per call)
@@ -1512,7 +1512,7 @@ def test_midgroup_random_shapes(pkg, dev, M, N, K, G, asym):
     (17, 2000, 4096, 512, True),       # two row tiles
     (32, 56, 6208, 128, True),         # one tile a group, 49 groups
     (33, 1000, 4160, 1024, True),      # four row tiles, a last K tile half padding
-    (64, 128, 27648, 1024, True),      # most rows, more groups a split than one
+    (64, 128, 27648, 1024, True),      # most rows, one workgroup of columns
 ])
 def test_midgroup_split_path(pkg, dev, M, N, K, G, asym):
     """Few rows with K split over workgroups: the reference's fp32 fold order bit for bit,
@@ -1544,6 +1544,23 @@ def test_midgroup_split_path(pkg, dev, M, N, K, G, asym):
         assert lib.w4a8_midgroup_gemm_split(a_hi.data_ptr(), a_lo.data_ptr(), a_scale.data_ptr(), a_ksum.data_ptr(),
                                             M, a_scale.stride(0), w_q.data_ptr(), 0, w_scale.data_ptr(),
                                             w_zero.data_ptr(), y1.data_ptr(), N, N, K, G, ptr, nbytes, stream) == 6
+
+
+@pytest.mark.parametrize("M,N,K,G,asym", [
+    (16, 5120, 8448, 128, True),       # one row tile: three or four one-tile groups a workgroup
+    (9, 2000, 8320, 128, False),       # one or two
+    (32, 5000, 6208, 128, True),       # two row tiles: two or three groups, the last half a tile
+    (24, 5120, 27648, 1024, True),     # one or two groups of eight tiles
+    (64, 4000, 6208, 128, True),       # four row tiles: three or four groups
+    (64, 5120, 10304, 512, False),     # one or two groups of four tiles, a short one last
+])
+def test_midgroup_split_several_groups(pkg, dev, M, N, K, G, asym):
+    """The same where a workgroup walks several groups: sums stored and cleared in mid-walk,
+    and odd numbers of tiles (the activation steps hold two)."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    groups, cols = pkg.geometry.num_groups(K, G), -(-N // 128)
+    assert groups > (2 if M > 32 else 3) * cus // cols, "one group a workgroup"
+    test_midgroup_split_path(pkg, dev, M, N, K, G, asym)
 
 
 def test_midgroup_split_rule(pkg):

@@ -20,8 +20,10 @@ activations, token scales, bf16 output)
 plus quant bytes 2*M*K + M*K + 2*M.  Inputs are resident in HBM before the
 timed region.  Per-shape kernel times (graph replays of back-to-back
 launches between HIP events), prefill TOPS and a CPU baseline
-(the reference's own C++ CPU GEMM on configs[0], timed on this host) are
-reported in the same JSON line.
+(the reference's own C++ CPU GEMM on configs[0], timed on this host) follow:
+a line each on stderr as they are measured, the rooflines and the CPU baseline in
+the JSON line too, every per-shape figure in the file that --detail-json names
+(the line stays short enough to be read whole from the end of a log).
 
     python bench.py [--gpus 1] [--steps 20] [--warmup 5]
 """
@@ -44,6 +46,10 @@ INT8_PEAK_TOPS = 5000.0        # MI355X dense int8 MFMA, TOP/s
 GROUP = 128
 DECODE_MS = (1, 4, 16, 64)
 PROJS = ("qkv_proj", "o_proj", "gate_up_proj", "down_proj")
+# the per-shape tables (about 22 KB of JSON), kept out of the printed line
+DETAIL_KEYS = ("decode_shapes", "stock_copy", "read_floor", "prefill_shapes", "int8_library_ref", "perchannel_shapes",
+               "config4_shapes", "compat_shapes", "tp4_shapes", "attention_shapes", "decoder",
+               "decoder_attention_kernel")
 
 
 def gemm_bytes(M, N, K, G=GROUP):
@@ -85,6 +91,8 @@ def main():
     ap.add_argument("--attention-sweep", action="store_true",
                     help="with the attention leg: also every split size (chunks per split 1-20) per concurrency")
     ap.add_argument("--no-detail", action="store_true", help="only the timed steps (for profiling)")
+    ap.add_argument("--detail-json", metavar="OUT",
+                    help="write the JSON line with every per-shape table to this file as well")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=10.0)
     ap.add_argument("--pmc-probe", action="store_true",
@@ -502,7 +510,9 @@ def main():
     # ---------------------------------------------------------------- CPU baseline
     if not args.no_cpu_baseline:
         result["cpu_baseline"] = cpu_baseline(pkg, dev, args.cpu_seconds)
-    print(json.dumps(result), flush=True)
+    if args.detail_json:
+        Path(args.detail_json).write_text(json.dumps(result, indent=1) + "\n")
+    print(json.dumps({k: v for k, v in result.items() if k not in DETAIL_KEYS}), flush=True)
 
 
 def config4(pkg, dev, synth, make_pool, time_graph, T):

@@ -2,10 +2,14 @@
 accept and refuse, and calls from several threads."""
 from __future__ import annotations
 
+import subprocess
+import sys
 import threading
 
 import pytest
 import torch
+
+from conftest import ROOT
 
 OPS = ["w4a8_quant_pertoken", "w4a8_gemm", "w4a8_gemm_swiglu", "w4a8_linear", "w4a8_rmsnorm_quant", "w4a8_rope_kv",
        "w4a8_attention", "w4a8_attention_rope", "midgroup_quant_a", "midgroup_w4a8_gemm", "midgroup_w4a8_gemm_tiled"]
@@ -16,6 +20,33 @@ def test_native_ops_are_registered(pkg):
     for op in OPS:
         assert torch._C._dispatch_has_kernel_for_dispatch_key(f"npu::{op}", "CUDA"), op
         assert not torch._C._dispatch_has_kernel_for_dispatch_key(f"npu::{op}", "CPU"), op
+
+
+@pytest.mark.parametrize("content", [None, b"not a library"])
+def test_host_side_without_the_native_ops(tmp_path, content):
+    """Without the ops' library, or with one this torch cannot load, the package imports, packs
+    weights on the CPU and keeps a CUDA kernel per op (one that raises)."""
+    lib = tmp_path / "w4a8_torch.so"
+    if content is not None:
+        lib.write_bytes(content)
+    code = f"""
+import importlib, importlib.util, pathlib, sys
+import torch
+import __graft_entry__ as g
+spec = importlib.util.spec_from_file_location(g.PKG_NAME, g.PKG_DIR / "__init__.py",
+                                              submodule_search_locations=[str(g.PKG_DIR)])
+pkg = importlib.util.module_from_spec(spec)
+sys.modules[g.PKG_NAME] = pkg
+importlib.import_module(g.PKG_NAME + "._abi").TORCH_LIB_PATH = pathlib.Path({str(lib)!r})
+spec.loader.exec_module(pkg)
+w_q, scale = pkg.packing.quantize_weight(torch.randn(32, 128), 64, torch.bfloat16)
+assert w_q.shape == (32, 64) and scale.shape == (2, 32)
+for op in {OPS!r}:
+    assert torch._C._dispatch_has_kernel_for_dispatch_key("npu::" + op, "CUDA"), op
+print("imported")
+"""
+    res = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0 and "imported" in res.stdout, res.stderr
 
 
 def _weight(dev, N, K, G, seed):

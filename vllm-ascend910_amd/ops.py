@@ -140,22 +140,31 @@ def _workspace(dev: torch.device, need: int) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------- C++ kernels
+def _without_native(error: type, why: str) -> None:
+    """The native ops raise when called; everything on the host works without them."""
+    def missing(*args, **kwargs):
+        raise error(f"{why}; build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+    for op in ("w4a8_quant_pertoken", "w4a8_gemm", "w4a8_gemm_swiglu", "w4a8_linear", "w4a8_rmsnorm_quant",
+               "w4a8_rope_kv", "w4a8_attention", "w4a8_attention_rope", "midgroup_quant_a", "midgroup_w4a8_gemm",
+               "midgroup_w4a8_gemm_tiled"):
+        _LIB.impl(op, missing, "CUDA")
+
+
 def _load_native() -> None:
     """Load csrc/torch_ops.cpp's library: importing it registers its ops' CUDA kernels.
-    Without it (not built) those ops raise FileNotFoundError when called."""
+    Not built, those ops raise FileNotFoundError when called; not loadable (built for another
+    torch, or this torch has no HIP), ImportError."""
     path = _abi.TORCH_LIB_PATH
     if not path.exists():
-        def missing(*args, **kwargs):
-            raise FileNotFoundError(f"W4A8 torch library not found at {path}; build it with "
-                                    f"`python -c 'import __graft_entry__ as g; g.build()'`")
-        for op in ("w4a8_quant_pertoken", "w4a8_gemm", "w4a8_gemm_swiglu", "w4a8_linear", "w4a8_rmsnorm_quant",
-                   "w4a8_rope_kv", "w4a8_attention", "w4a8_attention_rope", "midgroup_quant_a", "midgroup_w4a8_gemm",
-                   "midgroup_w4a8_gemm_tiled"):
-            _LIB.impl(op, missing, "CUDA")
+        _without_native(FileNotFoundError, f"W4A8 torch library not found at {path}")
         return
-    spec = importlib.util.spec_from_file_location("w4a8_torch", str(path))
-    native = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(native)
+    try:
+        spec = importlib.util.spec_from_file_location("w4a8_torch", str(path))
+        native = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(native)
+    except ImportError as e:
+        _without_native(ImportError, f"W4A8 torch library {path} cannot be loaded ({e})")
+        return
 
     def addresses():
         # the C ABI library, loaded at the first call of an op

@@ -180,8 +180,8 @@ def test_linear_bias_left_to_torch(pkg, dev):
 
 
 def test_which_biases_the_op_adds(pkg):
-    """Plain bf16 [N] tensors; none that autograd, forward mode or a function transform (vmap:
-    one GEMM for all biases) has to see."""
+    """Plain bf16 [N] tensors; none that autograd, forward mode or a function transform has to
+    see."""
     import torch.autograd.forward_ad as fwd
     takes = pkg.linear.__globals__["_epilogue_bias"]
     x, b = torch.zeros((2, 8), dtype=torch.bfloat16), torch.zeros((4,), dtype=torch.bfloat16)
@@ -203,9 +203,63 @@ def test_which_biases_the_op_adds(pkg):
     torch.func.vmap(torch.func.grad(record))(torch.stack([b, b]))
     torch.func.grad(record)(b)
     torch.func.jvp(record, (b,), (b,))
-    with torch.no_grad():
-        torch.func.vmap(record)(torch.stack([b, b]))
-    assert seen == [False] * 5
+    assert seen == [False] * 4
+
+
+def test_vmap_over_the_linear(pkg):
+    """Biases are batched on one product (nested too); other operands run one by one.  The op's
+    kernel stands in as a float product here."""
+    calls = []
+
+    def product(x, w_tiles, s_tiles, N, K, group, bias=None):
+        calls.append(tuple(x.shape))
+        y = (x.float() @ w_tiles.float()).to(torch.bfloat16)
+        return y if bias is None else y + bias
+
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn((3, 8), generator=g).to(torch.bfloat16)
+    w = torch.randn((2, 8, 4), generator=g).to(torch.bfloat16)
+    b = torch.randn((5, 2, 4), generator=g).to(torch.bfloat16)
+    s = torch.zeros(1)
+    with torch.library._scoped_library("npu", "IMPL") as lib:
+        lib.impl("w4a8_linear", product, "CPU")
+
+        def f(x, w, b):
+            return pkg.linear(x, w, s, 4, 128, b)
+
+        each = torch.stack([f(x, w[0], t) for t in b[:, 0]])
+        calls.clear()
+        assert torch.equal(torch.func.vmap(lambda t: f(x, w[0], t))(b[:, 0]), each)
+        assert torch.equal(torch.func.vmap(lambda t: f(x, w[0], t), in_dims=1)(b[:, 0].t().contiguous()), each)
+        nested = torch.func.vmap(torch.func.vmap(lambda t: f(x, w[0], t)))(b)
+        assert torch.equal(nested[:, 0], each)
+        assert calls == [(3, 8)] * 3
+        op = torch.ops.npu.w4a8_linear            # the op's own rule, as traced calls take it
+        assert torch.equal(torch.func.vmap(lambda t: op(x, w[0], s, 4, 8, 128, t))(b[:, 0]), each)
+        assert calls == [(3, 8)] * 4
+        got = torch.func.vmap(f, in_dims=(None, 0, 0))(x, w, b[0])
+        assert torch.equal(got, torch.stack([f(x, w[i], b[0, i]) for i in range(2)]))
+        got = torch.func.vmap(lambda x: f(x, w[0], None))(torch.stack([x, -x]))
+        assert torch.equal(got, torch.stack([f(x, w[0], None), f(-x, w[0], None)]))
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_traces_into_one_graph(pkg, bias):
+    """torch.compile takes the whole linear, bias included, as one op call."""
+    x = torch.randn((70, 256)).to(torch.bfloat16)
+    w, s = torch.zeros((4 * 2 * 1024,), dtype=torch.uint8), torch.zeros((4, 2, 16), dtype=torch.bfloat16)
+    b = torch.zeros((64,), dtype=torch.bfloat16) if bias else None
+    graphs = []
+
+    def backend(gm, example_inputs):
+        graphs.append([str(n.target) for n in gm.graph.nodes if n.op == "call_function"])
+        return gm.forward
+
+    torch._dynamo.reset()
+    fn = torch.compile(lambda x: pkg.linear(x, w, s, 64, 128, b), fullgraph=True, backend=backend)
+    with pytest.raises(NotImplementedError):     # traced, then run on the CPU, where the op has no kernel
+        fn(x)
+    assert graphs == [["npu.w4a8_linear"]]
 
 
 @pytest.mark.gpu

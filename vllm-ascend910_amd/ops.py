@@ -286,6 +286,18 @@ def _linear_fake(x, w_tiles, s_tiles, N, K, group, bias=None):
     return x.new_empty((x.shape[0], N), dtype=torch.bfloat16)
 
 
+@torch.library.register_vmap("npu::w4a8_linear", lib=_LIB)
+def _linear_vmap(info, in_dims, x, w_tiles, s_tiles, N, K, group, bias=None):
+    """Batched biases are added to one product; any other batched operand runs per element."""
+    op = torch.ops.npu.w4a8_linear
+    args = (x, w_tiles, s_tiles, N, K, group, bias)
+    dims = tuple(in_dims) + (None,) * (len(args) - len(in_dims))
+    if all(d is None for d in dims[:-1]):
+        return op(*args[:-1]) + bias.movedim(dims[-1], 0)[:, None], 0
+    each = [op(*(a if d is None else a.select(d, i) for a, d in zip(args, dims))) for i in range(info.batch_size)]
+    return torch.stack(each), 0
+
+
 # ---------------------------------------------------------------- RMSNorm + quant
 @torch.library.register_fake("npu::w4a8_rmsnorm_quant")
 def _rmsnorm_quant_fake(x, weight, eps, residual=None, group=0, want_normed=False):

@@ -640,7 +640,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const AttnArgs a) {
 // chunk there are 32 MFMAs (16 cycles each) and about 95 vector instructions off
 // the diagonal (16 exponentials at two issue slots), 32 more where a row's
 // maximum moves; 40 heads of 128 over 8 KV heads, one sequence: 4096 tokens
-// 283 -> 192 us, 0.90 PFLOP/s where a large bf16 matrix
+// 278 -> 195 us, 0.88 PFLOP/s where a large bf16 matrix
 // product reaches 1.19 on the same card.  What it took: two row tiles per wave
 // (one operand read serves two), masks only on the chunks that need them, lane
 // swaps instead of LDS permutes.  Slower at 4096 tokens: the softmax of one tile

@@ -493,8 +493,8 @@ __global__ __launch_bounds__(64 * kShWaves) void gemm_midgroup_shared_kernel(con
 // I[g][row][ldi]; mid_fold_kernel then folds the groups in the reference's order.
 // Without it the activation planes bound these shapes: every pair of column blocks
 // reads them again (16 rows: as many bytes as its weights), on as few workgroups
-// as N has column pairs.  27648 x 5120 at 16 rows: 32.6 us before, now 18.4 (the weights
-// at 3.8 TB/s) + 5.3 for the fold.
+// as N has column pairs.  27648 x 5120 at 16 rows: 32.6 us before, now 17.0 (the weights
+// at 4.2 TB/s) + 5.2 for the fold.
 constexpr int kSpP(int mt) { return mt == 1 ? 4 : 2; }   // activation steps in flight
 
 template <int MT>

@@ -82,10 +82,10 @@ __device__ __forceinline__ void zero_pads(int8_t* qr, int K, const PadMap& pm) {
 // so the per-element work spreads over gridDim.y CUs.  Rows past VPT * NT units
 // (SPLIT only) are read in a loop instead, and the workgroup's own units again.
 //
-// Bound by memory on many rows (16384 x 27648: 259 -> 231 us, 5.9 TB/s of its 1.36
+// Bound by memory on many rows (16384 x 27648: 253 -> 229 us, 5.9 TB/s of its 1.36
 // GB, from six instead of fourteen vector instructions per element) and by
 // latency on few: one memory round trip, two block-wide steps and the per-element
-// work of a thread's units (1 x 5120 3.1 -> 2.6 us in a graph of back-to-back calls).
+// work of a thread's units (1 x 5120 3.1 -> 2.5 us in a graph of back-to-back calls).
 template <int VPT, int NT, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(NT) void quant_act_vec_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int8_t* __restrict__ aq, int64_t lda,

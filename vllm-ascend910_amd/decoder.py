@@ -39,7 +39,8 @@ embeddings, RMSNorm) on this build's ops:
   returned in fp32.  Measured on MI355X (graph replays, one layer's decode
   attention at position 1100 of a 1280-position cache, us): kernel / products
   / SDPA 10.6 / 25 / 60 at 1 sequence, 14.8 / 28 / 65 at 8, 53.9 / 120 / 93 at
-  64; prefill of one 1024-token sequence 24.0 / 233 / 94.5;
+  64; prefill of one 1024-token sequence, a graph of one call, 33.8 / 233 / 104
+  (the kernel 25 back to back, 30 inside a layer);
 * the decode step is shape-static -- position, RoPE row, KV write index and
   mask are device tensors -- so it is captured once per batch size in a HIP
   graph and replayed, the greedy token feeding the next step inside the graph.

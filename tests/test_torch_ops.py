@@ -96,10 +96,10 @@ def test_rows_pass_through_by_their_strides(pkg):
     """Only contiguous rows K apart pass through; every other view comes out that way."""
     x = torch.randn((3, 64)).to(torch.bfloat16)
     rows = pkg.linear.__globals__["_rows"]
-    assert rows(x) is x
+    assert rows(x, 64) is x
     cases = list(_row_views(x[0]).values()) + [x.t().contiguous().t(), x.float(), x.view(1, 3, 64), x[:, :32], x[:0]]
     for v in cases:
-        got = rows(v)
+        got = rows(v, v.shape[-1])
         assert got.dtype is torch.bfloat16 and got.stride() == (v.shape[-1], 1) and got.is_contiguous()
         assert torch.equal(got, v.reshape(-1, v.shape[-1]).to(torch.bfloat16))
 

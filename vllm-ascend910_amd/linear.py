@@ -22,14 +22,14 @@ from . import ops  # noqa: F401  (registers torch.ops.npu.*)
 from .packing import quantize_weight
 
 
-def _rows(x: torch.Tensor) -> torch.Tensor:
-    """x as contiguous bf16 rows [M, K]; an activation that already is one passes through.
+def _rows(x: torch.Tensor, K: int) -> torch.Tensor:
+    """x [..., K] as contiguous bf16 rows [M, K]; an activation that already is one passes through.
 
-    (By its strides: is_contiguous() ignores a single row's, and the kernels take the row
-    stride as it is -- an expanded or transposed row would have one below K.)"""
-    if x.dim() == 2 and x.dtype is torch.bfloat16 and x.stride() == (x.shape[1], 1):
+    (By its strides, two of which make it 2-D: is_contiguous() ignores a single row's, and the
+    kernels take the row stride as it is -- an expanded or transposed row would have one below K.)"""
+    if x.dtype is torch.bfloat16 and x.stride() == (K, 1):
         return x
-    return x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
+    return x.reshape(-1, K).to(torch.bfloat16).contiguous()
 
 
 def _epilogue_bias(bias: torch.Tensor, x: torch.Tensor, N: int) -> bool:
@@ -53,7 +53,7 @@ def linear(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor, N: int
     """
     K = x.shape[-1]
     fused = bias is not None and _epilogue_bias(bias, x, N)
-    y = torch.ops.npu.w4a8_linear(_rows(x), w_tiles, s_tiles, N, K, group, bias if fused else None)
+    y = torch.ops.npu.w4a8_linear(_rows(x, K), w_tiles, s_tiles, N, K, group, bias if fused else None)
     if bias is not None and not fused:
         y = y + bias
     return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
@@ -67,7 +67,7 @@ def linear_swiglu(x: torch.Tensor, w_tiles: torch.Tensor, s_tiles: torch.Tensor,
     reference decoder layer's MLP activation (npu_ops/python/bench_decode_layer.py:78-81).
     """
     K = x.shape[-1]
-    a_q, a_scale = torch.ops.npu.w4a8_quant_pertoken(_rows(x), group)
+    a_q, a_scale = torch.ops.npu.w4a8_quant_pertoken(_rows(x, K), group)
     y = torch.ops.npu.w4a8_gemm_swiglu(a_q, a_scale, w_tiles, s_tiles, N, K, group)
     return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N // 2)
 
@@ -134,7 +134,8 @@ def midgroup_linear(x: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, wk: tor
     The reference's ``w4a8_ops.linear`` (npu_ops/python/w4a8_ops.py:243-252): quant_a pads the
     rows to TILE_M, so y has >= x's rows and is sliced before reshaping.
     """
-    K, x2 = x.shape[-1], _rows(x)
+    K = x.shape[-1]
+    x2 = _rows(x, K)
     a_hi, a_lo, a_scale, a_ksum = torch.ops.npu.midgroup_quant_a(x2, group)
     # only the real rows (the reference slices them from the padded product)
     y = torch.ops.npu.midgroup_w4a8_gemm(a_hi, a_lo, a_scale, a_ksum, wq, ws, wk, wz, K, group, x2.shape[0])
@@ -193,7 +194,8 @@ class MidGroupW4A8Linear(nn.Module):
         if self._gn is None:
             raise RuntimeError("MidGroupW4A8Linear: call process_weights_after_loading() after loading weights")
         ws, wk, wz = self._gn
-        k, x2 = x.shape[-1], _rows(x)
+        k = x.shape[-1]
+        x2 = _rows(x, k)
         rows = x2.shape[0]
         a_hi, a_lo, a_scale, a_ksum = torch.ops.npu.midgroup_quant_a(x2, self.group)
         if self._tiles is not None and self._tiles.device == x2.device:
